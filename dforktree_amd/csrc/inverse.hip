@@ -1,0 +1,169 @@
+// Standalone in-place (I+A)^-1 (fc1_block_inverse.py): one wave per matrix.
+//
+// The matrix (n <= NP = 16, 32 or 64) sits in LDS, NP x NP floats, and is
+// replaced there 16-row block by 16-row block, top down.  With X held as
+// 16 x 16 tiles, xt[i][j][r] of lane (n, g) = X[16i + n][16j + 4g + r]:
+//   X_ij <- E_ij - sum_{m = j}^{i-1} A_im X_mj   (fp32 MFMA 16x16x4, formed
+//           transposed, so that the product comes out in this layout)
+//   X_ij <- (I + A_ii)^-1 X_ij                   (forward substitution)
+// Step m of the substitution takes row m of every column from lane m of each
+// 16-lane row (one DPP row broadcast, fused into the multiply-add) and each
+// lane's own A[16i + n][16i + m], so the tiles of a block row share one
+// register per step and run side by side.  The sums are the forward
+// substitution's own, with no product by an inverted diagonal block.
+//
+// Bound by memory: 2 n^2 floats per matrix.  2048 64 x 64 matrices (67 MB),
+// with the copy that keeps the input (about 8 us): 44.5 us with one column
+// per lane (each lane read its own 256-byte row, element by element, and ran
+// 2016 dependent multiply-adds), 23.8 us here.  16 KiB of LDS at 64 nodes
+// holds 10 waves per CU, so 2048 matrices are resident at once.
+#include "dft_device.h"
+
+namespace dft {
+namespace {
+
+// 16-byte chunk c / 4 of row i at chunk position (c / 4) ^ i (mod the row's
+// chunks): rows stay contiguous, so one 1 KiB global->LDS load fills whole
+// rows, and the 16-byte reads of 16 rows at one column hit distinct banks
+// (at 64; 2- and 4-way conflicts at 32 and 16, where there are few reads).
+template <int NP>
+__device__ __forceinline__ int mat_at(int i, int c) {
+  return i * NP + ((((c >> 2) ^ i) & (NP / 4 - 1)) << 2) + (c & 3);
+}
+
+// Step M of the substitution on one tile: x[r] += na * (x[r] of lane M of the
+// 16-lane row).  The compiler keeps the broadcast as a move of its own (with
+// two wait states after each multiply-add), hence the statement; the two
+// wait states a DPP read needs after a vector write lie in the s_nop for the
+// first instruction and in the three others for the rest.  x must not come
+// straight from an MFMA: the backend does not see the reads in here.
+template <int M>
+__device__ __forceinline__ void subst_step(float na, f32x4& x) {
+  float x0 = x[0], x1 = x[1], x2 = x[2], x3 = x[3];
+  asm("s_nop 1\n\t"
+      "v_fmac_f32_dpp %0, %0, %4 row_newbcast:%c5 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %1, %1, %4 row_newbcast:%c5 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %2, %2, %4 row_newbcast:%c5 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %3, %3, %4 row_newbcast:%c5 row_mask:0xf bank_mask:0xf"
+      : "+v"(x0), "+v"(x1), "+v"(x2), "+v"(x3)
+      : "v"(na), "i"(M));
+  x = f32x4{x0, x1, x2, x3};
+}
+
+// steps M .. 14 on tiles 0 .. J - 1 of a block row
+template <int M, int J>
+__device__ __forceinline__ void subst_steps(const float (&na)[16], f32x4 (&x)[J]) {
+  if constexpr (M < 15) {
+#pragma unroll
+    for (int j = 0; j < J; ++j) subst_step<M>(na[M], x[j]);
+    subst_steps<M + 1, J>(na, x);
+  }
+}
+
+// block row I; xr[m][j]: X_mj of the block rows above as MFMA operands
+// (element s of lane (n, g): X[16m + 4g + s][16j + n])
+template <int NP, int I>
+__device__ __forceinline__ void block_rows(float* a, int n16, int g4, f32x4 (&xr)[NP / 16][NP / 16]) {
+  if constexpr (I < NP / 16) {
+    f32x4 x[I + 1];
+    if constexpr (I > 0) {
+      f32x4 am[I];  // A[16I + n][16m + 4g ..]
+#pragma unroll
+      for (int m = 0; m < I; ++m) am[m] = *reinterpret_cast<const f32x4*>(&a[mat_at<NP>(16 * I + n16, 16 * m + 4 * g4)]);
+#pragma unroll
+      for (int j = 0; j < I; ++j) {
+        x[j] = f32x4{};
+#pragma unroll
+        for (int m = j; m < I; ++m)
+#pragma unroll
+          for (int s = 0; s < 4; ++s) x[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(xr[m][j][s], am[m][s], x[j], 0, 0, 0);
+        x[j] = -x[j];
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x[I][r] = (n16 == 4 * g4 + r) ? 1.f : 0.f;
+    float na[16];  // the strict lower part of row n of A_II, negated
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(&a[mat_at<NP>(16 * I + n16, 16 * I + 4 * c)]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) na[4 * c + e] = 4 * c + e < n16 ? -v[e] : 0.f;
+    }
+    subst_steps<0, I + 1>(na, x);
+    // over A's rows 16I .., which nothing reads any more (one wave: its LDS
+    // operations run in order)
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int j = 0; j <= I; ++j) *reinterpret_cast<f32x4*>(&a[mat_at<NP>(16 * I + n16, 16 * j + 4 * g4)]) = x[j];
+    asm volatile("" ::: "memory");
+    if constexpr (I + 1 < NP / 16) {
+#pragma unroll
+      for (int j = 0; j <= I; ++j)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) xr[I][j][s] = a[mat_at<NP>(16 * I + 4 * g4 + s, 16 * j + n16)];
+    }
+    block_rows<NP, I + 1>(a, n16, g4, xr);
+  }
+}
+
+// VEC: n == NP and every matrix 16-byte aligned (whole 16-byte pieces, the
+// loads straight into LDS); else row by row, a column per lane.
+template <int NP, bool VEC>
+__global__ void __launch_bounds__(64) block_inverse_kernel(float* x, int n, int64_t mat_stride) {
+  __shared__ alignas(16) float a[NP * NP];
+  constexpr int CH = NP / 4;  // 16-byte chunks of a row
+  float* m = x + (int64_t)blockIdx.x * mat_stride;
+  const int lane = threadIdx.x;
+  if constexpr (VEC) {
+#pragma unroll
+    for (int b = 0; b < NP * NP / 256; ++b) {  // 1 KiB: rows (64 / CH) b ..
+      const int i = (64 / CH) * b + lane / CH;
+      __builtin_amdgcn_global_load_lds(m + i * NP + 4 * ((lane ^ i) & (CH - 1)),
+                                       (__attribute__((address_space(3))) void*)(a + 256 * b), 16, 0, 0);
+    }
+  } else {
+#pragma unroll 16
+    for (int i = 0; i < NP; ++i) {
+      const float v = (i < n && lane < n) ? m[i * n + lane] : 0.f;
+      if (lane < NP) a[mat_at<NP>(i, lane)] = v;
+    }
+  }
+  __syncthreads();
+  f32x4 xr[NP / 16][NP / 16];
+  block_rows<NP, 0>(a, lane & 15, lane >> 4, xr);
+  // tiles above the diagonal still hold A: zeros
+  if constexpr (VEC) {
+#pragma unroll
+    for (int b = 0; b < NP * NP / 256; ++b) {
+      const int i = (64 / CH) * b + lane / CH, c = (lane ^ i) & (CH - 1);
+      const f32x4 v = *reinterpret_cast<const f32x4*>(&a[256 * b + 4 * lane]);
+      *reinterpret_cast<f32x4*>(m + i * NP + 4 * c) = (c >> 2) > (i >> 4) ? f32x4{} : v;
+    }
+  } else {
+    if (lane < n)
+      for (int i = 0; i < n; ++i) m[i * n + lane] = (lane >> 4) > (i >> 4) ? 0.f : a[mat_at<NP>(i, lane)];
+  }
+}
+
+template <int NP>
+void launch(float* x, int n_mats, int n, int64_t mat_stride, hipStream_t stream) {
+  const bool vec = n == NP && reinterpret_cast<uintptr_t>(x) % 16 == 0 && mat_stride % 4 == 0;
+  if (vec)
+    hipLaunchKernelGGL((block_inverse_kernel<NP, true>), dim3(n_mats), dim3(64), 0, stream, x, n, mat_stride);
+  else
+    hipLaunchKernelGGL((block_inverse_kernel<NP, false>), dim3(n_mats), dim3(64), 0, stream, x, n, mat_stride);
+}
+
+}  // namespace
+
+int launch_block_inverse(float* x, int n_mats, int n, int64_t mat_stride, hipStream_t stream) {
+  if (n <= 16)
+    launch<16>(x, n_mats, n, mat_stride, stream);
+  else if (n <= 32)
+    launch<32>(x, n_mats, n, mat_stride, stream);
+  else
+    launch<64>(x, n_mats, n, mat_stride, stream);
+  return hipGetLastError() == hipSuccess ? DFT_OK : DFT_ERR_LAUNCH;
+}
+
+}  // namespace dft

@@ -305,39 +305,6 @@ __device__ __forceinline__ f32x4 mfma_f32_16x16x4(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// Forward substitution on one 32-node block held in registers:
-// x[i] -= A[base+i][base+m] x[m] for m < i (at[m][i] = A[i][m], pitch LDA).
-template <int LDA>
-__device__ __forceinline__ void solve_block32(float (&x)[32], const float* at, int base) {
-#pragma unroll
-  for (int m = 0; m < 31; ++m) {
-    const float xm = x[m];
-#pragma unroll
-    for (int i = m + 1; i < 32; ++i) x[i] -= at[(base + m) * LDA + base + i] * xm;
-  }
-}
-
-// y[i] -= sum_m A[ib+i][mb+m] x[m] (an off-diagonal 32x32 block)
-template <int LDA>
-__device__ __forceinline__ void update_block32(float (&y)[32], const float (&x)[32], const float* at, int mb, int ib) {
-#pragma unroll
-  for (int m = 0; m < 32; ++m) {
-    const float xm = x[m];
-#pragma unroll
-    for (int i = 0; i < 32; ++i) y[i] -= at[(mb + m) * LDA + ib + i] * xm;
-  }
-}
-
-// Forces x to be computed here: without a use at this point the compiler may
-// sink pure register arithmetic below a following barrier while the loads it
-// consumes stay above it, leaving every loaded operand live at once.
-__device__ __forceinline__ void materialize32(const float (&x)[32]) {
-#pragma unroll
-  for (int i = 0; i < 32; i += 8)
-    asm volatile("" ::"v"(x[i]), "v"(x[i + 1]), "v"(x[i + 2]), "v"(x[i + 3]), "v"(x[i + 4]), "v"(x[i + 5]),
-                 "v"(x[i + 6]), "v"(x[i + 7]));
-}
-
 // 8 bf16 as two 8-byte halves (columns c0..c0+3 and c0+16..c0+19 of a row)
 __device__ __forceinline__ bf16x8 lds_bf16x8_split(const uint16_t* first, const uint16_t* second) {
   const uint2 lo = *reinterpret_cast<const uint2*>(first);
@@ -2805,54 +2772,6 @@ int launch_tree_commit_verify(const dft_verify_args* a, const dft_pending_commit
       DFT_FUSED(32, grid, block, narrow)
   }
 #undef DFT_FUSED
-  return hipGetLastError() == hipSuccess ? DFT_OK : DFT_ERR_LAUNCH;
-}
-
-// ---------------------------------------------------------------------------
-// standalone in-place (I+A)^-1 (fc1_block_inverse.py): one wave per matrix,
-// lane j solves (I+A) x = e_j by forward substitution with column j in registers.
-// ---------------------------------------------------------------------------
-template <int NP>
-__global__ void __launch_bounds__(64) block_inverse_kernel(float* x, int n, int64_t mat_stride) {
-  constexpr int LD = NP + 4;
-  __shared__ float at[NP * LD];  // at[m][i] = A[i][m], strict lower part only
-  float* m = x + (int64_t)blockIdx.x * mat_stride;
-  const int lane = threadIdx.x;
-  if (lane < NP)
-    for (int mm = 0; mm < NP; ++mm)
-      at[mm * LD + lane] = (lane < n && mm < n && mm < lane) ? m[lane * n + mm] : 0.f;
-  __syncthreads();
-  float c0[32], c1[32];
-#pragma unroll
-  for (int i = 0; i < 32; ++i) {
-    c0[i] = (i == lane) ? 1.f : 0.f;
-    c1[i] = (i + 32 == lane) ? 1.f : 0.f;
-  }
-  solve_block32<LD>(c0, at, 0);
-  materialize32(c0);
-  if constexpr (NP == 64) {
-    update_block32<LD>(c1, c0, at, 0, 32);
-    solve_block32<LD>(c1, at, 32);
-    materialize32(c1);
-  }
-  __syncthreads();
-  if (lane < n) {
-#pragma unroll
-    for (int i = 0; i < 32; ++i)
-      if (i < n) m[i * n + lane] = c0[i];
-    if constexpr (NP == 64) {
-#pragma unroll
-      for (int i = 0; i < 32; ++i)
-        if (i + 32 < n) m[(i + 32) * n + lane] = c1[i];
-    }
-  }
-}
-
-int launch_block_inverse(float* x, int n_mats, int n, int64_t mat_stride, hipStream_t stream) {
-  if (n <= 32)
-    hipLaunchKernelGGL(block_inverse_kernel<32>, dim3(n_mats), dim3(64), 0, stream, x, n, mat_stride);
-  else
-    hipLaunchKernelGGL(block_inverse_kernel<64>, dim3(n_mats), dim3(64), 0, stream, x, n, mat_stride);
   return hipGetLastError() == hipSuccess ? DFT_OK : DFT_ERR_LAUNCH;
 }
 
