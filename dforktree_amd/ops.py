@@ -725,7 +725,13 @@ def packbits(x: torch.Tensor, bitorder: str = "little", *, out: Optional[torch.T
     semantics; returns the ceil(x.numel() / 8) bytes.  With `out` the bytes
     are written into it (no allocation; bytes past its end are dropped and
     `status` is set to 1)."""
-    dev = _device_of(x, out, status)
+    return _packbits(x, bitorder, out, status)
+
+
+def _packbits(x, bitorder, out, status=None, out_indptr=None):
+    """packbits; out_indptr (a contiguous int32 / int64 tensor of two entries)
+    receives [0, bytes] from the launch itself."""
+    dev = _device_of(x, out, status, out_indptr)
     xb = _byte_view(x, "x")
     nbytes = (xb.numel() + 7) // 8
     o = _out_bytes(out, nbytes, dev)
@@ -733,6 +739,8 @@ def packbits(x: torch.Tensor, bitorder: str = "little", *, out: Optional[torch.T
     a.n_segments, a.bit_order = 1, _bit_order(bitorder)
     a.x, a.n = xb.data_ptr(), xb.numel()
     a.out, a.out_capacity = o.data_ptr(), o.numel()
+    if out_indptr is not None:
+        a.out_indptr, a.out_indptr_dtype = out_indptr.data_ptr(), _itag(out_indptr, "out_indptr")
     a.status = _ptr(status)
     if xb.numel():
         check("dft_packbits", load().dft_packbits(C.byref(a), _stream(dev)))

@@ -60,8 +60,15 @@ def pack_mask_into(wrapper, mask: torch.Tensor, n_queries: int, kv_len: int) -> 
     buf = wrapper._custom_mask_buf
     if buf.numel() < nbytes:
         raise ValueError(f"custom mask needs {nbytes} bytes, the plan buffer holds {buf.numel()}")
-    _ops.packbits(mask.reshape(-1), "little", out=buf[:nbytes])
     ind = wrapper._mask_indptr_buf
+    # the launch writes [0, bytes] itself where it can: copied from the host,
+    # the two entries were a blocking copy per step (32.8 us a call for a 64 x
+    # 32795 mask, 12.4 us without and with the packing kernel's wide loads)
+    if (mask.is_cuda and nbytes and mask.numel() == n_queries * kv_len and ind.shape == (2,) and ind.is_contiguous()
+            and ind.dtype in (torch.int32, torch.int64) and ind.device == mask.device):
+        _ops._packbits(mask.reshape(-1), "little", buf[:nbytes], out_indptr=ind)
+        return nbytes
+    _ops.packbits(mask.reshape(-1), "little", out=buf[:nbytes])
     ind.copy_(torch.tensor([0, nbytes], dtype=ind.dtype, device=ind.device), non_blocking=True)
     return nbytes
 

@@ -136,3 +136,68 @@ def test_plan_override_packs_on_the_device(cuda, monkeypatch):
         assert int(w._custom_mask_buf[nbytes:].sum().item()) == 0
     finally:
         fake_flashinfer.remove_fakes(saved)
+
+
+# the elements start 0-5 bytes past an aligned address (whole dwords, shifted
+# dwords), the bytes 0-17 past one (cut words and 16-byte pieces at both ends)
+@pytest.mark.parametrize("x_off,out_off", [(0, 0), (1, 0), (2, 3), (3, 16), (4, 1), (5, 7)])
+@pytest.mark.parametrize("bitorder", ["little", "big"])
+def test_packbits_alignment(cuda, x_off, out_off, bitorder):
+    from dforktree_amd import ops
+    g = torch.Generator().manual_seed(17 * x_off + out_off)
+    for n in [1, 31, 32, 33, 39, 40, 41, 63, 64, 65, 255, 1023, 8193 * 8 - 1]:
+        announce(f"packbits alignment n={n} x+{x_off} out+{out_off} {bitorder}")
+        vals = torch.randint(0, 2, (n,), generator=g, dtype=torch.uint8) * torch.randint(1, 256, (n,), generator=g,
+                                                                                         dtype=torch.uint8)
+        x = torch.full((n + 16,), 255, dtype=torch.uint8, device=cuda)  # ones around the elements
+        x[x_off:x_off + n] = vals.to(cuda)
+        nbytes = (n + 7) // 8
+        buf = torch.full((nbytes + 64,), 0xA5, dtype=torch.uint8, device=cuda)
+        ops.packbits(x[x_off:x_off + n], bitorder, out=buf[out_off:out_off + nbytes])
+        got = buf.cpu().numpy()
+        assert np.array_equal(got[out_off:out_off + nbytes], M.packbits(vals.numpy(), bitorder)), n
+        assert (got[:out_off] == 0xA5).all() and (got[out_off + nbytes:] == 0xA5).all(), n
+
+
+@pytest.mark.parametrize("out_off", [0, 1, 4, 15])
+@pytest.mark.parametrize("bitorder", ["little", "big"])
+def test_tree_mask_alignment(cuda, out_off, bitorder):
+    """Segments at every byte alignment, rows shorter and longer than a 16-byte piece, one workgroup and many."""
+    from dforktree_amd import ops
+    sizes = [1, 2, 3, 31, 64, 33, 5, 64, 16]
+    kinds = ["chain", "bushy", "random"] * 3
+    parents, ancs = _batch(9, sizes, kinds)
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(sizes)]), dtype=torch.int32).to(cuda)
+    par = torch.tensor(np.concatenate(parents), dtype=torch.int32).to(cuda)
+    bits = ops.tree_struct(par, 4, cu_seqlens=cu, n_nodes=64, batch=len(sizes), want=("anc_bits",))["anc_bits"]
+    for plens in ([0] * 9, [0, 1, 126, 127, 128, 129, 255, 64, 63], [9000, 1, 40000, 3, 8191, 8192, 0, 20000, 70001]):
+        announce(f"tree mask alignment out+{out_off} {bitorder} prefixes {plens}")
+        want, want_ip = M.tree_masks_packed(ancs, plens, bitorder)
+        buf = torch.full((len(want) + 64,), 0xA5, dtype=torch.uint8, device=cuda)
+        out, ip = ops.tree_mask_pack(bits, torch.tensor(plens, device=cuda), cu_seqlens=cu, bitorder=bitorder,
+                                     out=buf[out_off:out_off + len(want)])
+        got = buf.cpu().numpy()
+        assert ip.cpu().numpy().tolist() == want_ip.tolist()
+        assert np.array_equal(got[out_off:out_off + len(want)], want)
+        assert (got[:out_off] == 0xA5).all() and (got[out_off + len(want):] == 0xA5).all()
+
+
+@pytest.mark.parametrize("form", ["int32", "int64", "strided", "two_rows"])
+def test_plan_indptr_forms(cuda, form):
+    """The wrapper's indptr buffer written by the launch (two contiguous
+    entries) or copied (any other form the copy broadcasts to)."""
+    import types
+    from dforktree_amd.plugin import fc1_plan as P
+    announce(f"plan indptr {form}")
+    n, plen = 16, 77
+    mask = torch.rand(n, plen + n, generator=torch.Generator().manual_seed(1)) > 0.5
+    ind = {"int32": torch.full((2,), -7, dtype=torch.int32, device=cuda),
+           "int64": torch.full((2,), -7, dtype=torch.int64, device=cuda),
+           "strided": torch.full((4,), -7, dtype=torch.int32, device=cuda)[::2],
+           "two_rows": torch.full((2, 2), -7, dtype=torch.int32, device=cuda)}[form]
+    w = types.SimpleNamespace(_custom_mask_buf=torch.zeros(1024, dtype=torch.uint8, device=cuda), _mask_indptr_buf=ind)
+    nbytes = P.pack_mask_into(w, mask.to(cuda), n, plen + n)
+    assert nbytes == (n * (plen + n) + 7) // 8
+    assert np.array_equal(w._custom_mask_buf[:nbytes].cpu().numpy(), M.packbits(mask.numpy()))
+    want = [0, nbytes]
+    assert ind.cpu().tolist() == ([want, want] if form == "two_rows" else want)
