@@ -1,28 +1,33 @@
 // Tree structure from parent indices (tree_ops.py:68-89, fc1_builder.py:38-47).
-// One wave per request (n <= 64 nodes, lane i = node i):
-//   - ancestor-or-self set of i as a uint64 (exact closure by a parent walk;
-//     the reference's five squarings stop at 31 edges, tree_ops.py:75-79),
+// One workgroup of four waves per request (n <= 64 nodes, lane i = node i):
+//   - ancestor-or-self set of i as a uint64 (exact closure by pointer
+//     doubling: after k rounds the set holds the ancestors at distances below
+//     2^k and p the 2^k-th one, so six rounds cover any tree; the reference's
+//     five squarings stop at 31 edges, tree_ops.py:75-79),
 //   - depth, conv gather columns cidx[i][kc-1-r] = kc-1 + (r-th ancestor)
 //     if r <= depth else kc-1-(r-depth) (tree_ops.py:81-88),
-//   - first child / next sibling links (fc1_builder.py:41-47).
+//   - first child / next sibling links (fc1_builder.py:41-47), from the set of
+//     every node's children.
 // Node 0 is the root; for i >= 1 the parent is max(parent[i], 0), the clamp
 // of tree_ops.py:73.  Integer work; results are bit-exact.
+//
+// Bound by the chain of one request: every wave forms the sets (registers
+// and lane shuffles), then wave 0 writes the sets, depths and status, wave 1
+// cidx, wave 2 the links, and all four the dense rows.  128 requests of 8-64
+// nodes with every output: 20.4 us with one wave per request that walked the
+// parents one LDS read at a time (63 for a chain) and searched the links by
+// a loop over the nodes, now 4.7 us.
 #include "dft_device.h"
 
 namespace dft {
 
-constexpr int kMaxKc = 16;
-
-__global__ void __launch_bounds__(256) tree_struct_kernel(const dft_tree_args p) {
-  __shared__ int spar[4][64];
+// One request.  A request whose parents form a cycle keeps what a walk of n
+// steps sees: the nodes it visits, depth n, status 2.
+__device__ __forceinline__ void tree_of_request(const dft_tree_args& p, int b, unsigned long long* kids) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int b = blockIdx.x * 4 + w;
-  const bool active = b < p.batch;  // every wave reaches the barrier below
-
-  int64_t row0 = 0;
-  int n = 0;
-  if (!active) {
-  } else if (p.cu_seqlens) {
+  int64_t row0;
+  int n;
+  if (p.cu_seqlens) {
     row0 = p.cu_seqlens[b];
     n = p.cu_seqlens[b + 1] - p.cu_seqlens[b];
   } else {
@@ -31,74 +36,77 @@ __global__ void __launch_bounds__(256) tree_struct_kernel(const dft_tree_args p)
   }
   n = n < 0 ? 0 : (n > 64 ? 64 : n);
   const int i = lane;
+  const bool in = i < n;
 
-  int status = 0;
-  int par = -1;
-  if (i < n && i > 0) {
+  bool bad = false;
+  int par = 0;  // (the root's: itself)
+  if (in && i > 0) {
     const int64_t raw = ld_i(p.parent, row0 + i, p.parent_dtype);
     par = raw < 0 ? 0 : (int)raw;
     if (par >= n) {  // out of range: treated as a child of the root
       par = 0;
-      status = 1;
+      bad = true;
     }
-    if (par >= i) status = 1;  // not topologically ordered
-  }
-  spar[w][i] = par;
-  __syncthreads();
-
-  uint64_t bits = 0;
-  int depth = 0;
-  int anc_r[kMaxKc];
-#pragma unroll
-  for (int r = 0; r < kMaxKc; ++r) anc_r[r] = 0;
-  if (i < n) {
-    bits = 1ull << i;
-    anc_r[0] = i;
-    int cur = i, steps = 0;
-    while (cur != 0 && steps < n) {
-      cur = spar[w][cur];
-      bits |= 1ull << cur;
-      ++depth;
-      ++steps;
-#pragma unroll
-      for (int r = 1; r < kMaxKc; ++r)
-        if (r == depth) anc_r[r] = cur;
-    }
-    if (cur != 0) status = 2;  // cycle
+    bad |= par >= i;  // not topologically ordered
   }
 
-  if (i < n) {
-    if (p.anc_bits) p.anc_bits[row0 + i] = bits;
-    if (p.depth) st_i(p.depth, row0 + i, p.depth_dtype, depth);
+  // (every lane takes part in the shuffles; lanes past the tree are no one's parent)
+  uint64_t bits = 1ull << i;
+  int up = par;
+#pragma unroll 1
+  for (int k = 0; k < 6 && __ballot(up != 0); ++k) {
+    bits |= __shfl(bits, up);
+    up = __shfl(up, up);
+  }
+  const bool cycle = up != 0;  // no root among 64 ancestors
+  if (!cycle) bits |= 1ull;
+  const int depth = cycle ? n : __popcll(bits) - 1;
+
+  if (w == 0) {
+    if (in) {
+      if (p.anc_bits) p.anc_bits[row0 + i] = bits;
+      if (p.depth) st_i(p.depth, row0 + i, p.depth_dtype, depth);
+    }
+    if (p.status) {
+      const uint64_t any_cycle = __ballot(in && cycle), any_bad = __ballot(in && bad);
+      if (lane == 0) p.status[b] = any_cycle ? 2 : (any_bad ? 1 : 0);
+    }
+  } else if (w == 1) {
     if (p.cidx) {
-      for (int r = 0; r < p.kc && r < kMaxKc; ++r) {
-        const int v = r <= depth ? (p.kc - 1 + anc_r[r]) : (p.kc - 1 - (r - depth));
-        st_i(p.cidx, (row0 + i) * p.kc + (p.kc - 1 - r), p.cidx_dtype, v);
+      int cur = i;  // the r-th ancestor
+      for (int r = 0; r < p.kc; ++r) {
+        const int v = r <= depth ? (p.kc - 1 + cur) : (p.kc - 1 - (r - depth));
+        if (in) st_i(p.cidx, (row0 + i) * p.kc + (p.kc - 1 - r), p.cidx_dtype, v);
+        cur = __shfl(par, cur);
       }
     }
-    if (p.nxt || p.sib) {
-      int nx = -1, sb = -1;
-      for (int v = n - 1; v > 0; --v)
-        if (spar[w][v] == i) nx = v;
-      for (int v = n - 1; v > i; --v)
-        if (spar[w][v] == par) sb = v;
-      if (p.nxt) st_i(p.nxt, row0 + i, p.link_dtype, nx);
-      if (p.sib) st_i(p.sib, row0 + i, p.link_dtype, sb);
+  } else if (w == 2 && (p.nxt || p.sib)) {
+    // (one wave: its LDS operations run in order)
+    volatile unsigned long long* k = kids;
+    k[i] = 0;
+    asm volatile("" ::: "memory");
+    if (in && i > 0) atomicOr(&kids[par], 1ull << i);
+    asm volatile("" ::: "memory");
+    const uint64_t own = k[i], later = k[par] & ~mask_upto(i);
+    if (in) {
+      if (p.nxt) st_i(p.nxt, row0 + i, p.link_dtype, own ? __ffsll((unsigned long long)own) - 1 : -1);
+      if (p.sib) st_i(p.sib, row0 + i, p.link_dtype, (i > 0 && later) ? __ffsll((unsigned long long)later) - 1 : -1);
     }
   }
-  if (!active) return;  // after the only barrier
   if (p.anc_f32) {
     // row r of the dense matrix: lane = column, coalesced
     float* base = p.anc_f32 + (int64_t)b * p.anc_req_stride;
-    for (int r = 0; r < n; ++r) {
-      const uint64_t rb = __shfl(bits, r);
-      if (lane < n) base[(int64_t)r * p.anc_row_stride + lane] = (float)((rb >> lane) & 1ull);
+    const uint32_t lo = (uint32_t)bits, hi = (uint32_t)(bits >> 32);
+    for (int r = w; r < n; r += 4) {  // (uniform)
+      const uint64_t rb = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, r) << 32) | (uint32_t)__builtin_amdgcn_readlane(lo, r);
+      if (in) base[(int64_t)r * p.anc_row_stride + lane] = (float)((rb >> lane) & 1ull);
     }
   }
-  if (p.status) {
-    const uint64_t bad1 = __ballot(status == 1), bad2 = __ballot(status == 2);
-    if (lane == 0) p.status[b] = bad2 ? 2 : (bad1 ? 1 : 0);
-  }
+}
+
+__global__ void __launch_bounds__(256) tree_struct_kernel(const dft_tree_args p) {
+  __shared__ unsigned long long kids[64];  // wave 2's
+  for (int b = blockIdx.x; b < p.batch; b += gridDim.x) tree_of_request(p, b, kids);
 }
 
 // Dense 0/1 ancestry rows -> the uint64 rows the verify and commit read.
@@ -137,7 +145,7 @@ int launch_anc_pack(const dft_anc_pack_args* a, hipStream_t stream) {
 }
 
 int launch_tree_struct(const dft_tree_args* a, hipStream_t stream) {
-  const dim3 grid((unsigned)((a->batch + 3) / 4));
+  const dim3 grid((unsigned)(a->batch < 65536 ? a->batch : 65536));  // workgroups stride over further requests
   hipLaunchKernelGGL(tree_struct_kernel, grid, dim3(256), 0, stream, *a);
   return hipGetLastError() == hipSuccess ? DFT_OK : DFT_ERR_LAUNCH;
 }

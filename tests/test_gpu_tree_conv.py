@@ -55,6 +55,63 @@ def test_tree_struct_status_flags(cuda):
     assert r["status"].cpu().tolist() == [1, 0, 2]
 
 
+def _walk(par, kc):
+    """A parent walk of at most n steps from every node: what the structure is for any parents, malformed ones too."""
+    n = len(par)
+    p = [0] + [max(int(v), 0) for v in par[1:]]
+    bad = any(v >= n or v >= i for i, v in enumerate(p) if i)
+    p = [v if v < n else 0 for v in p]
+    bits, depth, cidx, cyclic = [], [], [], False
+    for i in range(n):
+        seen, path, cur = 1 << i, [i], i
+        while cur != 0 and len(path) <= n:
+            cur = p[cur]
+            seen |= 1 << cur
+            path.append(cur)
+        cyclic |= cur != 0
+        d = len(path) - 1
+        bits.append(seen)
+        depth.append(d)
+        cidx.append([kc - 1 + path[r] if r <= d else kc - 1 - (r - d) for r in range(kc - 1, -1, -1)])
+    nxt = [next((v for v in range(1, n) if p[v] == i), -1) for i in range(n)]
+    sib = [next((v for v in range(i + 1, n) if i and p[v] == p[i]), -1) for i in range(n)]
+    return bits, depth, cidx, nxt, sib, 2 if cyclic else int(bad)
+
+
+@pytest.mark.parametrize("kc", [1, 4, 16])
+@pytest.mark.parametrize("dt", [torch.int32, torch.int64])
+def test_tree_struct_any_parents(cuda, kc, dt):
+    """Chains, cycles, self-parents, parents out of order and out of range, every size, packed with an empty request
+    and one longer than 64 nodes."""
+    from dforktree_amd import ops
+    announce(f"tree_struct any parents kc={kc} {dt}")
+    rng = np.random.default_rng(kc)
+    trees = [np.arange(n) - 1 for n in (1, 2, 3, 31, 32, 33, 63, 64)]                      # chains
+    trees += [np.concatenate([[-1], np.roll(np.arange(1, n), 1)]) for n in (2, 3, 33, 64)]  # one cycle
+    trees += [np.array([-1] + [int(rng.integers(-3, n + 3)) for _ in range(n - 1)]) for n in range(1, 65)]
+    trees += [np.array([-1] + [int(rng.integers(0, i)) for i in range(1, n)]) for n in range(1, 65)]
+    trees.insert(5, np.zeros(0, np.int64))
+    trees.insert(9, np.arange(70) - 1)  # cut to 64
+    cu = np.concatenate([[0], np.cumsum([len(t) for t in trees])])
+    r = ops.tree_struct(torch.tensor(np.concatenate(trees), dtype=dt).to(cuda), kc, n_nodes=64, batch=len(trees),
+                        cu_seqlens=torch.tensor(cu, dtype=torch.int32).to(cuda), index_dtype=dt)
+    torch.cuda.synchronize()
+    h = {k: v.cpu().numpy() for k, v in r.items()}
+    for b, t in enumerate(trees):
+        n, sl = min(len(t), 64), slice(cu[b], cu[b] + min(len(t), 64))
+        bits, depth, cidx, nxt, sib, status = _walk(t[:n], kc)
+        assert h["anc_bits"].view(np.uint64)[sl].tolist() == bits, b
+        assert h["depth"][sl].tolist() == depth, b
+        assert h["cidx"][sl].tolist() == cidx, b
+        assert h["nxt"][sl].tolist() == nxt and h["sib"][sl].tolist() == sib, b
+        assert int(h["status"][b]) == status, b
+        want = np.zeros((64, 64), np.float32)
+        for i in range(n):
+            want[i, :n] = [(bits[i] >> j) & 1 for j in range(n)]
+        assert np.array_equal(h["anc"][b], want), b
+    assert (h["anc_bits"][cu[9] + 64:cu[10]] == 0).all()
+
+
 def test_builder_tree_struct_matches_reference_closure(cuda):
     """builder.tree_struct (the opt-in for tree_ops.tree_struct) == the
     reference's squaring closure for N <= 32."""
