@@ -148,6 +148,7 @@ class MaskArgs(C.Structure):
 DFT_BITS_LITTLE, DFT_BITS_BIG = 0, 1
 
 EXPORTS = ("dft_tree_verify", "dft_tree_commit_verify", "dft_tree_conv", "dft_tree_commit", "dft_tree_struct",
+           "dft_tree_struct_filled",
            "dft_anc_pack", "dft_block_inverse", "dft_packbits", "dft_tree_mask_pack", "dft_size_order",
            "dft_error_string", "dft_abi_version")
 
@@ -179,6 +180,7 @@ def load() -> C.CDLL:
                        ("dft_tree_conv", [C.POINTER(ConvArgs), vp]),
                        ("dft_tree_commit", [C.POINTER(CommitArgs), vp]),
                        ("dft_tree_struct", [C.POINTER(TreeArgs), vp]),
+                       ("dft_tree_struct_filled", [C.POINTER(TreeArgs), i64, vp]),
                        ("dft_anc_pack", [C.POINTER(AncPackArgs), vp]),
                        ("dft_packbits", [C.POINTER(PackbitsArgs), vp]),
                        ("dft_tree_mask_pack", [C.POINTER(MaskArgs), vp]),

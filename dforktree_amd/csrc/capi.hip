@@ -11,7 +11,7 @@ int launch_block_inverse(float* x, int n_mats, int n, int64_t mat_stride, hipStr
 int launch_size_order(const int32_t* cu_seqlens, int batch, int n_nodes, int32_t* order, hipStream_t stream);
 int launch_tree_conv(const dft_conv_args* a, hipStream_t stream);
 int launch_tree_commit(const dft_commit_args* a, hipStream_t stream);
-int launch_tree_struct(const dft_tree_args* a, hipStream_t stream);
+int launch_tree_struct(const dft_tree_args* a, int64_t rows, hipStream_t stream);
 int launch_anc_pack(const dft_anc_pack_args* a, hipStream_t stream);
 int launch_packbits(const dft_packbits_args* a, hipStream_t stream);
 int launch_tree_mask(const dft_mask_args* a, hipStream_t stream);
@@ -54,6 +54,20 @@ int verify_status(const dft_verify_args* a, bool commit_only = false) {
   if (a->o_dtype != DFT_F32 && a->o_dtype != DFT_BF16 && a->o_dtype != DFT_F16) return DFT_ERR_INVALID;
   // q/k/v rows are copied as 16-byte pieces
   if (!aligned16(a->y) || a->y_row_stride % 8 != 0) return DFT_ERR_INVALID;
+  return DFT_OK;
+}
+
+// Checks shared by the tree-structure entry points (as verify_status).
+int tree_status(const dft_tree_args* a) {
+  if (!a) return DFT_ERR_INVALID;
+  if (a->batch < 0 || a->n_nodes < 0 || a->n_nodes > 64) return DFT_ERR_INVALID;
+  if (a->kc < 0 || a->kc > 16) return DFT_ERR_UNSUPPORTED;
+  if (a->batch == 0) return -1;
+  if (((int64_t)a->batch + 3) / 4 > max_blocks(256)) return DFT_ERR_UNSUPPORTED;
+  if (!a->parent || !index_tag(a->parent_dtype)) return DFT_ERR_INVALID;
+  if (a->depth && !index_tag(a->depth_dtype)) return DFT_ERR_INVALID;
+  if (a->cidx && (!index_tag(a->cidx_dtype) || a->kc < 1)) return DFT_ERR_INVALID;
+  if ((a->nxt || a->sib) && !index_tag(a->link_dtype)) return DFT_ERR_INVALID;
   return DFT_OK;
 }
 
@@ -162,16 +176,16 @@ int dft_tree_commit(const dft_commit_args* a, void* stream) {
 }
 
 int dft_tree_struct(const dft_tree_args* a, void* stream) {
-  if (!a) return DFT_ERR_INVALID;
-  if (a->batch < 0 || a->n_nodes < 0 || a->n_nodes > 64) return DFT_ERR_INVALID;
-  if (a->kc < 0 || a->kc > 16) return DFT_ERR_UNSUPPORTED;
-  if (a->batch == 0) return DFT_OK;
-  if (((int64_t)a->batch + 3) / 4 > max_blocks(256)) return DFT_ERR_UNSUPPORTED;  // a wave per request
-  if (!a->parent || !index_tag(a->parent_dtype)) return DFT_ERR_INVALID;
-  if (a->depth && !index_tag(a->depth_dtype)) return DFT_ERR_INVALID;
-  if (a->cidx && (!index_tag(a->cidx_dtype) || a->kc < 1)) return DFT_ERR_INVALID;
-  if ((a->nxt || a->sib) && !index_tag(a->link_dtype)) return DFT_ERR_INVALID;
-  return dft::launch_tree_struct(a, static_cast<hipStream_t>(stream));
+  const int st = tree_status(a);
+  if (st != DFT_OK) return st < 0 ? DFT_OK : st;
+  return dft::launch_tree_struct(a, -1, static_cast<hipStream_t>(stream));
+}
+
+int dft_tree_struct_filled(const dft_tree_args* a, int64_t rows, void* stream) {
+  const int st = tree_status(a);
+  if (st != DFT_OK) return st < 0 ? DFT_OK : st;
+  if (rows < 0) return DFT_ERR_INVALID;
+  return dft::launch_tree_struct(a, rows, static_cast<hipStream_t>(stream));
 }
 
 int dft_anc_pack(const dft_anc_pack_args* a, void* stream) {

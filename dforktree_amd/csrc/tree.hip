@@ -23,7 +23,11 @@ namespace dft {
 
 // One request.  A request whose parents form a cycle keeps what a walk of n
 // steps sees: the nodes it visits, depth n, status 2.
-__device__ __forceinline__ void tree_of_request(const dft_tree_args& p, int b, unsigned long long* kids) {
+// FILL: also zeroes the dense matrix outside the tree (n_nodes x n_nodes; a
+// tree cut to 64 rows is cut to n_nodes there) and the ancestry rows between
+// this request's last node and the next request.
+template <bool FILL>
+__device__ __forceinline__ void tree_of_request(const dft_tree_args& p, int b, int64_t rows_all, unsigned long long* kids) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   int64_t row0;
   int n;
@@ -34,6 +38,7 @@ __device__ __forceinline__ void tree_of_request(const dft_tree_args& p, int b, u
     row0 = (int64_t)b * p.n_nodes;
     n = p.n_nodes;
   }
+  const int span = n;
   n = n < 0 ? 0 : (n > 64 ? 64 : n);
   const int i = lane;
   const bool in = i < n;
@@ -97,16 +102,43 @@ __device__ __forceinline__ void tree_of_request(const dft_tree_args& p, int b, u
     // row r of the dense matrix: lane = column, coalesced
     float* base = p.anc_f32 + (int64_t)b * p.anc_req_stride;
     const uint32_t lo = (uint32_t)bits, hi = (uint32_t)(bits >> 32);
-    for (int r = w; r < n; r += 4) {  // (uniform)
-      const uint64_t rb = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, r) << 32) | (uint32_t)__builtin_amdgcn_readlane(lo, r);
-      if (in) base[(int64_t)r * p.anc_row_stride + lane] = (float)((rb >> lane) & 1ull);
+    const int rows = FILL ? p.n_nodes : n, cols = rows;
+    for (int r = w; r < rows; r += 4) {  // (uniform)
+      uint64_t rb = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, r) << 32) | (uint32_t)__builtin_amdgcn_readlane(lo, r);
+      if (FILL && r >= n) rb = 0;
+      if (lane < cols) base[(int64_t)r * p.anc_row_stride + lane] = (float)((rb >> lane) & 1ull);
     }
   }
+  if (FILL && p.anc_bits)
+    for (int64_t r = row0 + 64 + threadIdx.x; r < row0 + span && r < rows_all; r += 256) p.anc_bits[r] = 0;
 }
 
-__global__ void __launch_bounds__(256) tree_struct_kernel(const dft_tree_args p) {
+// FILL: the grid's last workgroup zeroes the ancestry rows (of `rows`) in
+// front of the first request and behind the last.
+template <bool FILL>
+__global__ void __launch_bounds__(256) tree_struct_kernel(const dft_tree_args p, int64_t rows) {
   __shared__ unsigned long long kids[64];  // wave 2's
-  for (int b = blockIdx.x; b < p.batch; b += gridDim.x) tree_of_request(p, b, kids);
+  const int stride = (int)gridDim.x - (FILL ? 1 : 0);
+  if (FILL && (int)blockIdx.x == stride) {
+    if (!p.anc_bits) return;
+    int64_t lo = 0, hi = (int64_t)p.batch * p.n_nodes;
+    if (p.cu_seqlens) {
+      __shared__ int ends[2];
+      if (threadIdx.x == 0) ends[0] = ends[1] = p.cu_seqlens[0];
+      __syncthreads();
+      for (int q = 1 + threadIdx.x; q <= p.batch; q += 256) {
+        atomicMin(&ends[0], p.cu_seqlens[q]);
+        atomicMax(&ends[1], p.cu_seqlens[q]);
+      }
+      __syncthreads();
+      lo = ends[0];
+      hi = ends[1] < 0 ? 0 : ends[1];
+    }
+    for (int64_t r = threadIdx.x; r < lo && r < rows; r += 256) p.anc_bits[r] = 0;
+    for (int64_t r = hi + threadIdx.x; r < rows; r += 256) p.anc_bits[r] = 0;
+    return;
+  }
+  for (int b = blockIdx.x; b < p.batch; b += stride) tree_of_request<FILL>(p, b, rows, kids);
 }
 
 // Dense 0/1 ancestry rows -> the uint64 rows the verify and commit read.
@@ -144,9 +176,13 @@ int launch_anc_pack(const dft_anc_pack_args* a, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? DFT_OK : DFT_ERR_LAUNCH;
 }
 
-int launch_tree_struct(const dft_tree_args* a, hipStream_t stream) {
-  const dim3 grid((unsigned)(a->batch < 65536 ? a->batch : 65536));  // workgroups stride over further requests
-  hipLaunchKernelGGL(tree_struct_kernel, grid, dim3(256), 0, stream, *a);
+// rows >= 0: the filling form over that many ancestry rows
+int launch_tree_struct(const dft_tree_args* a, int64_t rows, hipStream_t stream) {
+  const unsigned grid = (unsigned)(a->batch < 65536 ? a->batch : 65536);  // workgroups stride over further requests
+  if (rows >= 0)
+    hipLaunchKernelGGL(tree_struct_kernel<true>, dim3(grid + 1), dim3(256), 0, stream, *a, rows);
+  else
+    hipLaunchKernelGGL(tree_struct_kernel<false>, dim3(grid), dim3(256), 0, stream, *a, rows);
   return hipGetLastError() == hipSuccess ? DFT_OK : DFT_ERR_LAUNCH;
 }
 

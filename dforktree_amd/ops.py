@@ -624,10 +624,10 @@ def tree_struct(parent: torch.Tensor, kc: int = 4, *, batch: Optional[int] = Non
     a.parent, a.parent_dtype = parent.data_ptr(), _itag(parent, "parent")
     a.cu_seqlens = _ptr(cu_seqlens)
     if "anc_bits" in want:
-        out["anc_bits"] = torch.zeros(rows, device=dev, dtype=torch.int64)
+        out["anc_bits"] = torch.empty(rows, device=dev, dtype=torch.int64)
         a.anc_bits = out["anc_bits"].data_ptr()
     if "anc" in want:
-        out["anc"] = torch.zeros(batch, n_nodes, n_nodes, device=dev, dtype=torch.float32)
+        out["anc"] = torch.empty(batch, n_nodes, n_nodes, device=dev, dtype=torch.float32)
         a.anc_f32, a.anc_row_stride, a.anc_req_stride = out["anc"].data_ptr(), n_nodes, n_nodes * n_nodes
     if "depth" in want:
         out["depth"] = torch.empty(rows, device=dev, dtype=index_dtype)
@@ -645,7 +645,10 @@ def tree_struct(parent: torch.Tensor, kc: int = 4, *, batch: Optional[int] = Non
     if "status" in want:
         out["status"] = torch.empty(batch, device=dev, dtype=torch.int32)
         a.status = out["status"].data_ptr()
-    check("dft_tree_struct", load().dft_tree_struct(C.byref(a), _stream(dev)))
+    if batch == 0 and "anc_bits" in want:
+        out["anc_bits"].zero_()  # (no launch)
+    # zeroes what no tree covers: two fill launches fewer per call
+    check("dft_tree_struct_filled", load().dft_tree_struct_filled(C.byref(a), rows, _stream(dev)))
     return out
 
 

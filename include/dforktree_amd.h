@@ -397,6 +397,12 @@ typedef struct dft_tree_args {
 
 DFT_API int dft_tree_struct(const dft_tree_args* args, void* stream);
 
+/* The same, for outputs that nothing has cleared: what no tree covers is
+ * zeroed by the launch, i.e. the rest of each dense n_nodes x n_nodes matrix
+ * (a request longer than n_nodes is cut to it there), and of anc_bits'
+ * `rows` entries those of no request and past a request's 64th node. */
+DFT_API int dft_tree_struct_filled(const dft_tree_args* args, int64_t rows, void* stream);
+
 /* ---------------------------------------------------------------------------
  * Dense ancestry to bit rows: anc_bits[b*n_nodes + i] bit j = (anc[b][i][j]
  * > 0.5) for j <= i (bits above the diagonal are dropped), n_nodes <= 64.

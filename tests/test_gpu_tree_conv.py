@@ -112,6 +112,34 @@ def test_tree_struct_any_parents(cuda, kc, dt):
     assert (h["anc_bits"][cu[9] + 64:cu[10]] == 0).all()
 
 
+@pytest.mark.parametrize("n_nodes", [3, 17, 64])
+def test_tree_struct_fills_what_no_tree_covers(cuda, n_nodes):
+    """Rows in front of, behind and between the requests, and the dense
+    matrices outside the trees, are zeros on memory that held something else;
+    a request past n_nodes stays inside its own matrix."""
+    from dforktree_amd import ops
+    announce(f"tree_struct fill n_nodes={n_nodes}")
+    sizes, lead, tail = [2, 0, n_nodes, 1, n_nodes + 9], 5, 300
+    cu = np.cumsum([lead] + sizes)
+    rows = int(cu[-1]) + tail
+    parent = torch.zeros(rows, dtype=torch.int32, device=cuda)  # stars
+    parent[cu[:-1].tolist()] = -1
+    for shape, dt in (((rows,), torch.int64), ((len(sizes), n_nodes, n_nodes), torch.float32)):
+        torch.full(shape, -3, dtype=dt, device=cuda)  # what the allocator hands out again
+    r = ops.tree_struct(parent, 4, cu_seqlens=torch.tensor(cu, dtype=torch.int32).to(cuda), n_nodes=n_nodes,
+                        batch=len(sizes), want=("anc_bits", "anc"))
+    bits, anc = r["anc_bits"].cpu().numpy(), r["anc"].cpu().numpy()
+    want = np.zeros(rows, np.uint64)
+    dense = np.zeros((len(sizes), n_nodes, n_nodes), np.float32)
+    for b, n in enumerate(sizes):
+        for i in range(min(n, 64)):
+            want[cu[b] + i] = (1 << i) | 1
+            if i < n_nodes:
+                dense[b, i, 0] = dense[b, i, i] = 1
+    assert np.array_equal(bits.view(np.uint64), want)
+    assert np.array_equal(anc, dense)
+
+
 def test_builder_tree_struct_matches_reference_closure(cuda):
     """builder.tree_struct (the opt-in for tree_ops.tree_struct) == the
     reference's squaring closure for N <= 32."""
