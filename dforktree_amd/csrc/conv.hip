@@ -54,8 +54,10 @@ __global__ void __launch_bounds__(256) tree_conv_kernel(const dft_conv_args p) {
   st_f(p.y, (int64_t)b * p.y_req_stride + (int64_t)n * p.y_node_stride + c, p.y_dtype, out);
 }
 
-// Fast path for the plugin's layout: width 4, bf16 tokens / weights / output
-// / window, channel-contiguous rows.  A block of one wave (64 threads)
+// The plugin's layout (width 4, bf16 tokens / weights / output / window,
+// channel-contiguous rows) where the conv state is of another type or a tree
+// has more than 64 nodes; tree_conv4_rows_kernel below takes the rest, and
+// the figures here are of the time when this kernel took it all.  A block of one wave (64 threads)
 // covers 512 channels of one node; a thread owns 8 consecutive channels, so every
 // gathered token row, the weights (8 channels x 4 taps) and the output are
 // 16-byte accesses.  The gather columns are uniform over the block: the four
@@ -214,6 +216,162 @@ __global__ void __launch_bounds__(64) tree_conv4_bf16_kernel(const dft_conv_args
   }
 }
 
+// The fast path's main form, for a bf16 conv state and trees of up to 64
+// nodes: a workgroup of 8 waves takes 256 channels of one request and holds
+// every column of [conv_state || x] in LDS (and a row of zeros for taps
+// outside it), 512 bytes each.  The token rows are copied in (two per 1 KiB
+// copy) without waiting for the tap columns and are read from memory once
+// instead of once per tap; a lane owns 4 channels, whose weights stay in
+// registers; a wave takes every 8th node of the workgroup's share and reads
+// the next node's columns ahead.
+//
+// A node's window over the slice (iw[n][c][0..2], 1.5 KiB) goes through LDS
+// and leaves as 16-byte pieces of whole lines, non-temporal: it is read back
+// for the accepted nodes only, and kept out of the caches it does not push
+// out the tokens and y (40 -> 37 us per launch; y is read by the verify that
+// follows, and stored past the caches too it made that pair slower: 83 -> 86
+// us at batch 64, although the conv alone took 30).
+//
+// 64 requests x 32 nodes x 8192 channels, six layers in turn (168 MB each):
+// 54.8 us per launch with a one-wave workgroup per node that gathered its
+// four rows from memory, 37.2 here, 4.5 TB/s; a streaming probe moves 5.2
+// TB/s at this mix of reads and writes.  The same rows in cache: 42.0 -> 32.8.
+// Batch 4: 8.2 -> 5.6, batch 1 (plugin step, 24 layers): 354 -> 334.  4 waves
+// took 1.2 us longer, 16 4 us.
+constexpr int kConvNodes = 64, kConvSlice = 256, kConvWaves = 8;
+
+// rows of the workgroup's LDS: zeros, 3 state columns, the tokens (an odd
+// count's last copy fills one more)
+__host__ __device__ constexpr int conv_rows(int n) { return 4 + n + (n & 1); }
+
+// 4 channels (of lane l) of the four rows at these byte offsets
+__device__ __forceinline__ void tap_rows(const uint16_t* rows, const int* taps, int n, int lane, uint2 (&r)[4]) {
+  const int4 t = *reinterpret_cast<const int4*>(&taps[4 * n]);
+  const char* base = reinterpret_cast<const char*>(rows) + 8 * lane;
+  r[0] = *reinterpret_cast<const uint2*>(base + t.x);
+  r[1] = *reinterpret_cast<const uint2*>(base + t.y);
+  r[2] = *reinterpret_cast<const uint2*>(base + t.z);
+  r[3] = *reinterpret_cast<const uint2*>(base + t.w);
+}
+
+template <bool CIDX64>
+__global__ void __launch_bounds__(64 * kConvWaves) tree_conv4_rows_kernel(const dft_conv_args p, int cblocks,
+                                                                          int splits) {
+  extern __shared__ u32x4 conv_lds[];
+  const int N = p.n_nodes;
+  uint16_t* rows = reinterpret_cast<uint16_t*>(conv_lds);                // [conv_rows(N)][256]
+  int* taps = reinterpret_cast<int*>(rows + conv_rows(N) * kConvSlice);  // [N][4] byte offsets into rows
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  uint16_t* stage = reinterpret_cast<uint16_t*>(taps + 4 * N) + wave * 3 * kConvSlice;  // the wave's window
+
+  // ids that agree mod 8 (one XCD) hold the node shares of a (request, slice)
+  const int id = blockIdx.x, k = id >> 3;
+  const int split = k % splits, pair = (k / splits) * 8 + (id & 7);
+  if (pair >= p.batch * cblocks) return;  // uniform over the workgroup
+  const int cb = pair % cblocks, b = pair / cblocks;
+  const int cbase = cb * kConvSlice, nch = min(kConvSlice, p.channels - cbase);  // a multiple of 8
+
+  // the slots (a negative state slot reads slot 0, a negative window slot writes no window)
+  const int64_t slot_raw = p.cs_indices ? req_index(p.cs_indices, p.cs_indices_dtype, b) : b;
+  const int64_t dst = p.iw_indices ? req_index(p.iw_indices, p.iw_indices_dtype, b) : b;
+  {
+    // (channels past the last read channel 0 of the slice instead)
+    const uint16_t* xb = static_cast<const uint16_t*>(p.x) + (int64_t)b * p.x_req_stride + cbase;
+    const int c8 = 8 * (lane & 31), half = lane >> 5;
+    for (int r = 2 * wave; r < N; r += 2 * kConvWaves)
+      __builtin_amdgcn_global_load_lds(xb + min(r + half, N - 1) * p.x_node_stride + (c8 < nch ? c8 : 0),
+                                       (__attribute__((address_space(3))) void*)(rows + (4 + r) * kConvSlice), 16, 0, 0);
+  }
+  if (tid < 4 * N) {
+    const int64_t at = (int64_t)b * p.cidx_req_stride + (int64_t)(tid >> 2) * p.cidx_node_stride + (tid & 3);
+    const int64_t col =
+        CIDX64 ? static_cast<const int64_t*>(p.cidx)[at] : (int64_t) static_cast<const int32_t*>(p.cidx)[at];
+    taps[tid] = col >= 0 && col < 3 + N ? 2 * kConvSlice * (1 + (int)col) : 0;
+  }
+  const int c0 = 4 * lane;
+  const bool active = c0 < nch;
+  float w[16];  // w[4 e + j]: channel c0 + e, tap j
+  {
+    const u32x4* wp = reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(p.weight) +
+                                                     (int64_t)(cbase + (active ? c0 : 0)) * 4);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const u32x4 u = wp[q];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        w[8 * q + 2 * e] = __uint_as_float(u[e] << 16);
+        w[8 * q + 2 * e + 1] = __uint_as_float(u[e] & 0xffff0000u);
+      }
+    }
+  }
+  float bias[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) bias[e] = p.bias && active ? ld_f(p.bias, cbase + c0 + e, p.bias_dtype) : 0.f;
+  if (tid < nch) {
+    const int64_t slot = slot_raw < 0 ? 0 : slot_raw;
+    const uint16_t* cs = static_cast<const uint16_t*>(p.conv_state) + slot * p.cs_slot_stride +
+                         (int64_t)(cbase + tid) * p.cs_chan_stride;
+    uint16_t h[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) h[j] = cs[j * p.cs_col_stride];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) rows[(1 + j) * kConvSlice + tid] = h[j];
+  }
+  if (tid < 64) *reinterpret_cast<uint2*>(rows + 4 * tid) = uint2{0u, 0u};
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the row copies
+  __syncthreads();
+
+  uint16_t* yb = static_cast<uint16_t*>(p.y) + (int64_t)b * p.y_req_stride + cbase + c0;
+  const bool window = p.iw && dst >= 0;
+  uint16_t* iwb = static_cast<uint16_t*>(p.iw) + dst * p.iw_slot_stride + 3 * cbase;
+  const int pieces = 3 * nch / 8;  // of a node's window
+  const int share = (N + splits - 1) / splits, n_end = min(N, (split + 1) * share);
+  int n = split * share + wave;
+  uint2 next[4] = {};
+  if (n < n_end) tap_rows(rows, taps, n, lane, next);
+  for (; n < n_end; n += kConvWaves) {
+    const uint2 r[4] = {next[0], next[1], next[2], next[3]};
+    if (n + kConvWaves < n_end) tap_rows(rows, taps, n + kConvWaves, lane, next);
+    float acc[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] = bias[e];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      acc[0] += __uint_as_float(r[j].x << 16) * w[j];
+      acc[1] += __uint_as_float(r[j].x & 0xffff0000u) * w[4 + j];
+      acc[2] += __uint_as_float(r[j].y << 16) * w[8 + j];
+      acc[3] += __uint_as_float(r[j].y & 0xffff0000u) * w[12 + j];
+    }
+    if (p.silu) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] = acc[e] / (1.f + expf(-acc[e]));
+    }
+    if (active) {
+      const bf16x2 lo = __builtin_convertvector((f32x2{acc[0], acc[1]}), bf16x2);  // round to nearest even
+      const bf16x2 hi = __builtin_convertvector((f32x2{acc[2], acc[3]}), bf16x2);
+      uint2 o;
+      __builtin_memcpy(&o.x, &lo, 4);
+      __builtin_memcpy(&o.y, &hi, 4);
+      *reinterpret_cast<uint2*>(yb + n * p.y_node_stride) = o;
+    }
+    if (window) {
+      // [channel][tap 1 .. 3]; a pair of channels is three words: (t1 t2) (t3 t1') (t2' t3')
+      uint2* st = reinterpret_cast<uint2*>(stage + 12 * lane);
+      const uint32_t a1 = r[1].x, a2 = r[2].x, a3 = r[3].x, b1 = r[1].y, b2 = r[2].y, b3 = r[3].y;
+      st[0] = uint2{__builtin_amdgcn_perm(a2, a1, 0x05040100u), __builtin_amdgcn_perm(a1, a3, 0x07060100u)};
+      st[1] = uint2{__builtin_amdgcn_perm(a3, a2, 0x07060302u), __builtin_amdgcn_perm(b2, b1, 0x05040100u)};
+      st[2] = uint2{__builtin_amdgcn_perm(b1, b3, 0x07060100u), __builtin_amdgcn_perm(b3, b2, 0x07060302u)};
+      asm volatile("" ::: "memory");  // (one wave: its LDS operations run in order)
+      const u32x4* sv = reinterpret_cast<const u32x4*>(stage);
+      const u32x4 v0 = sv[lane], v1 = sv[64 + (lane & 31)];
+      u32x4* iw = reinterpret_cast<u32x4*>(iwb + n * p.iw_node_stride);
+      if (lane < pieces) __builtin_nontemporal_store(v0, iw + lane);
+      if (lane < 32 && 64 + lane < pieces) __builtin_nontemporal_store(v1, iw + 64 + lane);
+      asm volatile("" ::: "memory");
+    }
+  }
+}
+
 static bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; }
 
 // The fast path needs the plugin's layout; anything else takes the
@@ -230,8 +388,30 @@ static bool conv4_bf16_ok(const dft_conv_args* a) {
   return true;
 }
 
+// A launch of few (request, slice) pairs divides each pair's nodes over
+// several workgroups, which each copy all rows in, until there is one per CU
+// or a wave has one node (batch 1: 334 us per plugin step, 375 undivided).
+// More nodes than the LDS rows hold, or a conv state of another type, take
+// the per-node kernel.
+static bool launch_conv4_rows(const dft_conv_args* a, hipStream_t stream) {
+  if (a->cs_dtype != DFT_BF16 || a->n_nodes > kConvNodes) return false;
+  const int cblocks = (a->channels + kConvSlice - 1) / kConvSlice;
+  const int64_t pairs8 = ((int64_t)a->batch * cblocks + 7) / 8;
+  int splits = 1;
+  while (splits * kConvWaves < a->n_nodes && pairs8 * 8 * splits < 256) splits *= 2;
+  if (pairs8 * 8 * splits > (int64_t)0xffffffffll / (64 * kConvWaves)) return false;  // work-items in 32 bits
+  const size_t lds = 2 * kConvSlice * (size_t)conv_rows(a->n_nodes) + 16 * a->n_nodes + 6 * kConvSlice * kConvWaves;
+  const dim3 grid((unsigned)(pairs8 * 8 * splits)), block(64 * kConvWaves);
+  if (a->cidx_dtype == DFT_I64)
+    hipLaunchKernelGGL(tree_conv4_rows_kernel<true>, grid, block, lds, stream, *a, cblocks, splits);
+  else
+    hipLaunchKernelGGL(tree_conv4_rows_kernel<false>, grid, block, lds, stream, *a, cblocks, splits);
+  return true;
+}
+
 int launch_tree_conv(const dft_conv_args* a, hipStream_t stream) {
-  if (conv4_bf16_ok(a)) {
+  if (conv4_bf16_ok(a) && launch_conv4_rows(a, stream)) {
+  } else if (conv4_bf16_ok(a)) {
     const int cblocks = (a->channels + 511) / 512;
     const int64_t pairs8 = ((int64_t)a->batch * cblocks + 7) / 8;
     const dim3 grid((unsigned)(pairs8 * 8 * a->n_nodes));

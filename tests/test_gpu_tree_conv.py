@@ -320,3 +320,37 @@ def test_anc_pack_matches_oracle_bits(cuda, n):
     torch.cuda.synchronize()
     assert np.array_equal(got.cpu().numpy(), want)
     assert np.array_equal(one.cpu().numpy(), want[n:2 * n])
+
+
+# nodes on both sides of a wave's and a workgroup's share and of the LDS rows'
+# limit, slices cut at 8 channels, taps outside [conv_state || x], each index
+# width; a float conv state takes the per-node kernel
+@pytest.mark.parametrize("cs_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,N,C", [(1, 1, 8), (1, 2, 256), (2, 7, 248), (1, 8, 264), (3, 9, 1000), (9, 16, 512),
+                                   (1, 31, 2048), (2, 33, 776), (70, 5, 1024), (1, 63, 264), (5, 64, 520),
+                                   (2, 65, 256)])
+def test_conv_slices(cuda, B, N, C, cs_dtype):
+    from dforktree_amd import ops
+    announce(f"conv slices B={B} N={N} C={C} {cs_dtype}")
+    g = torch.Generator().manual_seed(1000 * N + C + B)
+    x = torch.randn(B, N, C, generator=g).to(torch.bfloat16)
+    w = (torch.randn(C, 4, generator=g) * 0.5).to(torch.bfloat16)
+    cs = torch.randn(B, C, 3, generator=g).to(cs_dtype)
+    cidx = torch.randint(-2, N + 6, (B, N, 4), generator=g)
+    bias = torch.randn(C, generator=g)
+    xt = torch.cat((cs.double().transpose(1, 2), x.double(), torch.zeros(B, 1, C, dtype=torch.float64)), 1)
+    cols = torch.where((cidx >= 0) & (cidx < N + 3), cidx, N + 3)
+    taps = torch.stack([xt[b][cols[b].reshape(-1)].view(N, 4, C) for b in range(B)])
+    acc = (taps * w.double().t()).sum(2) + bias.double()
+    want, win = acc / (1 + (-acc).exp()), taps[:, :, 1:].transpose(2, 3).to(torch.bfloat16)
+    for it in (torch.int32, torch.int64):
+        y = torch.full((B * N * C + 64,), 7.0, dtype=torch.bfloat16, device=cuda)
+        iw = torch.full((B * N * C * 3 + 64,), 7.0, dtype=torch.bfloat16, device=cuda)
+        ops.tree_conv(x.to(cuda), cs.to(cuda), w.to(cuda), bias.to(cuda), cidx.to(it).to(cuda),
+                      y=y[:B * N * C].view(B, N, C), iw=iw[:B * N * C * 3].view(B, N, C, 3))
+        got = y[:B * N * C].view(B, N, C).cpu().double()
+        # half a bf16 unit of the result, and the fp32 sum's and SiLU's rounding
+        bound = want.abs() * 2.0 ** -8 + 1e-5 * ((taps.abs() * w.double().abs().t()).sum(2) + bias.double().abs())
+        assert bool(((got - want).abs() <= bound).all())
+        assert torch.equal(iw[:B * N * C * 3].view(B, N, C, 3).cpu(), win)
+        assert bool((y[B * N * C:] == 7).all()) and bool((iw[B * N * C * 3:] == 7).all())  # nothing past the slices
