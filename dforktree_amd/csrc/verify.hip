@@ -580,20 +580,22 @@ struct PathKeys<NW, true> {
 // of the recompute, the rows of W's accumulator layout; vr[e][t]: tile t's
 // column, two bf16 per register), with the gain and b gate of position
 // lane % 16.
-template <int NW, bool RVN>
+// (NWC: column waves of the item, over all its workgroups)
+template <int NWC, bool RVN>
 struct PathVals {
-  float v[4][Waves<NW>::TT];
+  float v[4][Waves<NWC>::TT];
   float g[4];
 };
-template <int NW>
-struct PathVals<NW, true> {
+template <int NWC>
+struct PathVals<NWC, true> {
   u16x2 vr[4];
   float gl, bl;
 };
-template <int NW, bool RAWK, bool RVN>
+template <int NW, int NWC, bool RAWK, bool RVN>
 __device__ __forceinline__ void issue_pending(const dft_pending_commit& c, const Pending& pd, int h, int wave, int lane,
-                                              const float* dummy, PathKeys<NW, RAWK>& pk, PathVals<NW, RVN>& pv) {
-  constexpr int KP = 8 / NW, TT = Waves<NW>::TT, CW = Waves<NW>::CW;
+                                              const float* dummy, PathKeys<NW, RAWK>& pk, PathVals<NWC, RVN>& pv,
+                                              int col0) {
+  constexpr int KP = 8 / NW, TT = Waves<NWC>::TT, CW = Waves<NWC>::CW;
   const bool any = pd.last >= 0;
   const int n16 = lane & 15, g4 = lane >> 4;
   const int krow = __shfl(pd.ent, 4 * (wave & 3) + g4);
@@ -621,7 +623,7 @@ __device__ __forceinline__ void issue_pending(const dft_pending_commit& c, const
     for (int e = 0; e < 4; ++e) {
       const int64_t row = __shfl(pd.ent, 4 * e + g4);  // slot 4g + e is position 4e + g
 #pragma unroll
-      for (int t = 0; t < TT; ++t) pv.vr[e][t] = vb[row * vs + CW * wave + 16 * t + n16];
+      for (int t = 0; t < TT; ++t) pv.vr[e][t] = vb[row * vs + col0 + CW * wave + 16 * t + n16];
     }
     pv.gl = gb[pd.ent * gs];
     // the b gate as the verify reads it: the whole 32-bit word, converted later
@@ -636,7 +638,7 @@ __device__ __forceinline__ void issue_pending(const dft_pending_commit& c, const
     for (int s = 0; s < 4; ++s) {
       const int row = __shfl(pd.ent, 4 * s + g4);
 #pragma unroll
-      for (int t = 0; t < TT; ++t) pv.v[s][t] = vb[row * vs + CW * wave + 16 * t + n16];
+      for (int t = 0; t < TT; ++t) pv.v[s][t] = vb[row * vs + col0 + CW * wave + 16 * t + n16];
       pv.g[s] = gb[row * gs];
     }
   }
@@ -680,10 +682,10 @@ __device__ __forceinline__ void issue_path_dma(const dft_pending_commit& c, cons
 }
 // The keys, gains and b gates issue_pending would have loaded, read from
 // those copies (the values are read where W is formed: path_values<VLDS>).
-template <int NW>
+template <int NW, int NWC>
 __device__ __forceinline__ void path_from_lds(const dft_pending_commit& c, const Pending& pd, int h, int wave,
                                               int lane, const uint16_t* praw, const float* rvx,
-                                              PathKeys<NW, true>& pk, PathVals<NW, true>& pv) {
+                                              PathKeys<NW, true>& pk, PathVals<NWC, true>& pv) {
   const int n16 = lane & 15, g4 = lane >> 4;
   const int rs = rvn_slot(4 * (wave & 3) + g4);
 #pragma unroll
@@ -851,11 +853,12 @@ __device__ __forceinline__ void mat16_store(float* D, f32x4 acc, int n16, int g4
 // when nothing is pending).
 // VLDS: the raw value rows are in LDS (rows 16 + position of the key
 // staging, issue_path_dma) rather than in pv.vr.
-template <int NW, bool RAWK, bool VLDS = false>
+template <int NWC, bool RAWK, bool VLDS = false>
 __device__ __forceinline__ void path_values(const Pending& pd, const float* pkey, float* rvx,
-                                            const PathVals<NW, true>& pv, int wave, int lane,
-                                            const f32x4 (&s0r)[Waves<NW>::TT][8], float (&vnr)[4][Waves<NW>::TT]) {
-  constexpr int TT = Waves<NW>::TT;
+                                            const PathVals<NWC, true>& pv, int wave, int lane,
+                                            const f32x4 (&s0r)[Waves<NWC>::TT][8], float (&vnr)[4][Waves<NWC>::TT],
+                                            int col0) {
+  constexpr int TT = Waves<NWC>::TT;
   const int n16 = lane & 15, g4 = lane >> 4;
 #pragma unroll
   for (int s = 0; s < 4; ++s)
@@ -976,7 +979,7 @@ __device__ __forceinline__ void path_values(const Pending& pd, const float* pkey
     const bool ok = (pd.vmask >> ip) & 1u;
 #pragma unroll
     for (int t = 0; t < TT; ++t) {
-      const uint16_t vb = VLDS ? reinterpret_cast<const uint16_t*>(pkey)[qkv_at(16 + ip, Waves<NW>::CW * wave + 16 * t + n16)]
+      const uint16_t vb = VLDS ? reinterpret_cast<const uint16_t*>(pkey)[qkv_at(16 + ip, col0 + Waves<NWC>::CW * wave + 16 * t + n16)]
                                : vr[e][t];
       w[t][e] = ok ? bp * (bf16_bits_to_f32(vb) - ep * w[t][e]) : 0.f;
     }
@@ -1008,11 +1011,12 @@ __device__ __forceinline__ void path_values(const Pending& pd, const float* pkey
 // the keys the staging waits for), or null for no walk check; a path that
 // fails it is dropped here (pd then says nothing is pending, and the caller
 // writes nothing back).
-template <int NW, bool LINES, bool RAWK, bool RVN, bool VLDS = false>
+template <int NW, int NWC, bool LINES, bool RAWK, bool RVN, bool VLDS = false>
 __device__ __forceinline__ void commit_tile(Pending& pd, float* pkey, float* rvx, const PathKeys<NW, RAWK>& kr,
-                                            const PathVals<NW, RVN>& pv, int wave, int lane,
-                                            f32x4 (&s0r)[Waves<NW>::TT][8], const uint32_t* walk, int bound) {
-  constexpr int TT = Waves<NW>::TT;
+                                            const PathVals<NWC, RVN>& pv, int wave, int lane,
+                                            f32x4 (&s0r)[Waves<NWC>::TT][8], const uint32_t* walk, int bound,
+                                            int col0) {
+  constexpr int TT = Waves<NWC>::TT;
   const int n16 = lane & 15, g4 = lane >> 4;
   stage_pending_keys<NW, RAWK, RVN>(pkey, rvx, kr, wave, lane);
   __syncthreads();
@@ -1020,7 +1024,7 @@ __device__ __forceinline__ void commit_tile(Pending& pd, float* pkey, float* rvx
     pd.last = -1;
     pd.vmask = 0;
   }
-  if constexpr (LINES) state_to_mfma<NW>(s0r, lane);
+  if constexpr (LINES) state_to_mfma<NWC>(s0r, lane);
   float gp[4], vnr[4][TT];
   if constexpr (RVN) {
     // The swapped tile in registers of its own: left to itself the compiler
@@ -1034,7 +1038,7 @@ __device__ __forceinline__ void commit_tile(Pending& pd, float* pkey, float* rvx
 #pragma unroll
         for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(s0r[t][j]));
     __builtin_amdgcn_sched_barrier(0);
-    path_values<NW, RAWK, VLDS>(pd, pkey, rvx, pv, wave, lane, s0r, vnr);
+    path_values<NWC, RAWK, VLDS>(pd, pkey, rvx, pv, wave, lane, s0r, vnr, col0);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int s = 0; s < 4; ++s) gp[s] = __shfl(pv.gl, 4 * s + g4);
@@ -1960,7 +1964,7 @@ __device__ __forceinline__ void fused_status(const Item& it, int lane, uint32_t 
 
 // The body of the one-head-per-workgroup kernels (COMMIT: the fused commit ->
 // verify form).
-// CS (plain verify of up to 32 nodes): the item's value columns are split
+// CS (up to 32 nodes, or the plain verify): the item's value columns are split
 // over CS workgroups, CS items apart in the grid's last dimension; each
 // forms phase 1 in full and phases 2-3 on its 128 / CS columns.
 // ---------------------------------------------------------------------------
@@ -2221,13 +2225,17 @@ __device__ __forceinline__ void verify_body(const VerifyParams& P, int tid_in, i
   constexpr bool kHalves = NP > 32 && CS > 1;
   constexpr int NWC = kHalves ? NW : NW * CS;  // column waves of the item (of all its workgroups)
   constexpr int TT = Waves<NWC>::TT, CW = Waves<NWC>::CW;
-  static_assert(CS == 1 || !COMMIT, "the column split serves the plain verify");
+  static_assert(CS == 1 || !COMMIT || NP == 32, "the column split serves the plain verify and the 32-wide fused forms");
   static_assert(!kHalves || (CS == 2 && S0VEC), "the 64-wide split takes two workgroups and a vector state");
   // The 32-wide fused form runs phase 1 (which needs no state) before its
   // commit, under the state stream, and stages the commit's keys and
   // write-back in the v region, whose rows it copies in afterwards.
   constexpr bool kEarly = COMMIT && !VerifySmem<NP>::kLateV;
-  constexpr int kPlanes = (VerifySmem<NP>::kLateV || kEarly) ? 2 : 3;  // the late forms copy v rows later
+  // The column-split fused forms (small launches, where LDS is not short)
+  // stage the commit in an array of its own, and the v rows come with the
+  // q/k rows instead of behind the write-back.
+  constexpr bool kStageApart = kEarly && CS > 1;
+  constexpr int kPlanes = (VerifySmem<NP>::kLateV || (kEarly && !kStageApart)) ? 2 : 3;  // the late forms copy v rows later
   // PDMA: the path's raw rows are copied into LDS ahead of the state tile
   // (16-byte aligned key and value rows; issue_path_dma)
   constexpr bool kPathDma = PDMA;
@@ -2256,12 +2264,24 @@ __device__ __forceinline__ void verify_body(const VerifyParams& P, int tid_in, i
     }
   }();
 
+  // the fused forms' commit staging: the v region, or (column split) 8 KiB apart
+  float* const cstage = [&]() -> float* {
+    if constexpr (kStageApart) {
+      __shared__ alignas(16) float apart[16 * kD];
+      return apart;
+    } else if constexpr (kEarly) {
+      return reinterpret_cast<float*>(sm.vrows());
+    } else {
+      return nullptr;
+    }
+  }();
+
   // (the wave index as a scalar: in a vector register it is held, and at the
   // fused form's register cap spilled, through phase 1)
   const int tid = tid_in, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n16 = lane & 15, g4 = lane >> 4;
 
-  if constexpr (!COMMIT && CS > 1) args_early(P);
+  if constexpr (CS > 1) args_early(P);
   Item it;
   int col0 = 0;  // the workgroup's first value column
   if constexpr (GIVEN) {
@@ -2294,18 +2314,18 @@ __device__ __forceinline__ void verify_body(const VerifyParams& P, int tid_in, i
       if (pd.last >= 0) {  // uniform (one request)
         f32x4 s0r[TT][8];
         PathKeys<NW, RAWK> kr;
-        PathVals<NW, RVN> pv;
+        PathVals<NWC, RVN> pv;
         // (the ancestry rows go first: the keys the commit waits for land behind them)
         issue_walk_dma<false>(P.c, pd, wave, lane, S0, walk);
-        issue_state<true, kEarly, NW>(S0, p.state_v_stride, wave, lane, s0r);
-        issue_pending<NW, RAWK, RVN>(P.c, pd, it.h, wave, lane, S0, kr, pv);
-        commit_tile<NW, kEarly, RAWK, RVN>(pd, sm.pkey(), rvx, kr, pv, wave, lane, s0r,
-                                           P.c.prev_anc_bits ? walk : nullptr, ph.bound);
+        issue_state<true, kEarly, NWC>(S0, p.state_v_stride, wave, lane, s0r);
+        issue_pending<NW, NWC, RAWK, RVN>(P.c, pd, it.h, wave, lane, S0, kr, pv, col0);
+        commit_tile<NW, NWC, kEarly, RAWK, RVN>(pd, sm.pkey(), rvx, kr, pv, wave, lane, s0r,
+                                                P.c.prev_anc_bits ? walk : nullptr, ph.bound, col0);
         __syncthreads();  // every wave has read the staged keys: am + x take the write-back staging
         if (pd.last >= 0)  // uniform: a path that is not a walk was dropped
-          store_state<NW>(const_cast<float*>(S0), p.state_v_stride, wave, lane, s0r, sm.amx + wave * 512);
+          store_state<NWC>(const_cast<float*>(S0), p.state_v_stride, wave, lane, s0r, sm.amx + wave * 512);
       }
-      if (it.h == 0 && wave == 0) fused_status(it, lane, word, walk);
+      if (it.h == 0 && wave == 0 && col0 == 0) fused_status(it, lane, word, walk);
       return;
     }
   }
@@ -2324,7 +2344,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& P, int tid_in, i
   // beside the tile, they would be spilled.)
   Pending pd{};
   PathKeys<NW, RAWK> kr;
-  PathVals<NW, RVN> pv;
+  PathVals<NWC, RVN> pv;
   uint32_t pword = 0;
   if constexpr (COMMIT && !kEarly) pword = *path_word(P.c, it.b, lane);
   if constexpr (kPathDma) {
@@ -2336,12 +2356,12 @@ __device__ __forceinline__ void verify_body(const VerifyParams& P, int tid_in, i
   issue_rows<NP, 0, kPlanes, NW>(p, it, wave, lane, sm);
   if constexpr (COMMIT && !kEarly) {
     pd = decode_pending(ph, lane, pword);
-    issue_pending<NW, RAWK, RVN>(P.c, pd, it.h, wave, lane, S0, kr, pv);
+    issue_pending<NW, NWC, RAWK, RVN>(P.c, pd, it.h, wave, lane, S0, kr, pv, col0);
     issue_walk_dma<false>(P.c, pd, wave, lane, S0, sm.graw[4]);  // (lands before the state, as the gates)
   }
   if constexpr (kPathDma) {
     const Pending pd0 = decode_pending(ph, lane, pword);
-    issue_path_dma<NW>(P.c, pd0, it.h, wave, lane, S0, reinterpret_cast<uint16_t*>(sm.vrows()), rvx);
+    issue_path_dma<NW>(P.c, pd0, it.h, wave, lane, S0, reinterpret_cast<uint16_t*>(cstage), rvx);
     issue_walk_dma<false>(P.c, pd0, wave, lane, S0, sm.graw[4]);
   }
   asm volatile("" ::: "memory");
@@ -2397,14 +2417,14 @@ __device__ __forceinline__ void verify_body(const VerifyParams& P, int tid_in, i
   phase_norms<NP, NW, (NP > 32 || CS > 1)>(p, tid, sm, sm);
   __syncthreads();
   if constexpr (COMMIT && !kEarly) {
-    commit_tile<NW, false, RAWK, RVN>(pd, sm.pkey(), rvx, kr, pv, wave, lane, s0r,
-                                      P.c.prev_anc_bits ? sm.graw[4] : nullptr, ph.bound);
+    commit_tile<NW, NWC, false, RAWK, RVN>(pd, sm.pkey(), rvx, kr, pv, wave, lane, s0r,
+                                           P.c.prev_anc_bits ? sm.graw[4] : nullptr, ph.bound, col0);
     // everything this wave loaded has been consumed: no load is left in
     // flight past the (conditional) write-back
     __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));
     if (pd.last >= 0) {  // uniform over the workgroup (one request)
       __syncthreads();  // every wave has read the staged keys: am + x take the write-back staging
-      store_state<NW>(const_cast<float*>(S0), p.state_v_stride, wave, lane, s0r, sm.amx + wave * 512);
+      store_state<NWC>(const_cast<float*>(S0), p.state_v_stride, wave, lane, s0r, sm.amx + wave * 512);
     }
     __syncthreads();  // am and x take the Gram tiles and X
   }
@@ -2419,13 +2439,13 @@ __device__ __forceinline__ void verify_body(const VerifyParams& P, int tid_in, i
   // 4-7; the 32-wide: waves 2-3).
   constexpr int kSaveWave0 = MT;
   const int mtn = (it.n + 15) >> 4;  // uniform over the workgroup
-  // (the plain verify with a vector state has registers for 3 rows ahead.
-  // The 32-wide fused forms, whose phase 1 runs under their state stream,
-  // keep the 16-lane solve: with the whole-wave one the headline form
+  // (the plain verify with a vector state and the column-split fused forms
+  // have registers for 3 rows ahead.  The other 32-wide fused forms, whose
+  // phase 1 runs under their state stream, keep the 16-lane solve: with the whole-wave one the headline form
   // measured 62.73 -> 63.13 us at batch 64, and the form holding raw path
   // rows in registers spilled.)
-  constexpr bool kWaveSolve = !kEarly;
-  phase_gram_diag<NP, NW, (!COMMIT && S0VEC) ? 3 : 1, kWaveSolve>(tid, sm, sm, mtn);
+  constexpr bool kWaveSolve = !kEarly || CS > 1;
+  phase_gram_diag<NP, NW, ((!COMMIT || CS > 1) && S0VEC) ? 3 : 1, kWaveSolve>(tid, sm, sm, mtn);
   if constexpr (!kEarly)
     if (wave >= kSaveWave0)
       phase_saves<NP, COMMIT, NW, VerifySmem<NP>, VerifySmem<NP>, CS, 64 * (NW - kSaveWave0)>(
@@ -2438,7 +2458,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& P, int tid_in, i
     pd = decode_pending(ph, lane, sm.graw[4][lane & 15]);
     if constexpr (!kPathDma) {
       issue_walk_dma<true>(P.c, pd, wave, lane, S0, sm.graw[4]);  // ahead of the path loads that cover it
-      issue_pending<NW, RAWK, RVN>(P.c, pd, it.h, wave, lane, S0, kr, pv);
+      issue_pending<NW, NWC, RAWK, RVN>(P.c, pd, it.h, wave, lane, S0, kr, pv, col0);
     }
   }
   if constexpr (kSplit && !kHalves) issue_state_group<COMMIT, kEarly, NWC>(S0, p.state_v_stride, wave, lane, 2, s0r);
@@ -2459,24 +2479,26 @@ __device__ __forceinline__ void verify_body(const VerifyParams& P, int tid_in, i
     if constexpr (!RVN) {
       pd = decode_pending(ph, lane, sm.graw[4][lane & 15]);
       issue_walk_dma<true>(P.c, pd, wave, lane, S0, sm.graw[4]);
-      issue_pending<NW, RAWK, RVN>(P.c, pd, it.h, wave, lane, S0, kr, pv);
+      issue_pending<NW, NWC, RAWK, RVN>(P.c, pd, it.h, wave, lane, S0, kr, pv, col0);
     }
-    float* stage = reinterpret_cast<float*>(sm.vrows());  // 8 KiB: the 16 path keys, then the write-back
+    float* stage = cstage;  // 8 KiB: the 16 path keys, then the write-back
     if constexpr (kPathDma)
-      path_from_lds<NW>(P.c, pd, it.h, wave, lane, reinterpret_cast<const uint16_t*>(stage), rvx, kr, pv);
-    commit_tile<NW, true, RAWK, RVN, kPathDma>(pd, stage, rvx, kr, pv, wave, lane, s0r,
-                                               P.c.prev_anc_bits ? sm.graw[4] : nullptr, ph.bound);
+      path_from_lds<NW, NWC>(P.c, pd, it.h, wave, lane, reinterpret_cast<const uint16_t*>(stage), rvx, kr, pv);
+    commit_tile<NW, NWC, true, RAWK, RVN, kPathDma>(pd, stage, rvx, kr, pv, wave, lane, s0r,
+                                                    P.c.prev_anc_bits ? sm.graw[4] : nullptr, ph.bound, col0);
     __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));
     if (pd.last >= 0) {  // uniform over the workgroup (one request)
       __syncthreads();  // every wave has read the staged keys
-      store_state<NW>(const_cast<float*>(S0), p.state_v_stride, wave, lane, s0r, stage + wave * 512);
+      store_state<NWC>(const_cast<float*>(S0), p.state_v_stride, wave, lane, s0r, stage + wave * 512);
     }
-    __syncthreads();  // every wave has read its staging back: the v region takes the v rows
-    // (row addresses recomputed from an opaque copy of the lane id: shared
-    // with the q/k copies at the start, they would be held through the commit)
-    int lane_v = lane;
-    asm volatile("" : "+v"(lane_v));
-    issue_rows<NP, 2, 3, NW>(p, it, wave, lane_v, sm);
+    if constexpr (!kStageApart) {
+      __syncthreads();  // every wave has read its staging back: the v region takes the v rows
+      // (row addresses recomputed from an opaque copy of the lane id: shared
+      // with the q/k copies at the start, they would be held through the commit)
+      int lane_v = lane;
+      asm volatile("" : "+v"(lane_v));
+      issue_rows<NP, 2, 3, NW>(p, it, wave, lane_v, sm);
+    }
   }
 
   f32x4 cq[MT][TT], ck[MT][TT];
@@ -2497,10 +2519,11 @@ __device__ __forceinline__ void verify_body(const VerifyParams& P, int tid_in, i
   } else {
     bf16x8 sh[4][TT], sl[4][TT];  // (unused: one pass)
     phase_cq_ck<NP, 3, NWC, 0>(lane, sm, s0r, cq, ck, mtn, sh, sl);
-    if constexpr (kEarly) __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));  // the v row copies (untracked)
+    if constexpr (kEarly && !kStageApart) __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));  // the v row copies (untracked)
     __syncthreads();  // X and Pq complete
   }
-  if constexpr (kEarly) phase_saves<NP, COMMIT, NW>(P, it, tid, sm, sm);  // the k rows are intact until phase 3
+  if constexpr (kEarly)  // the k rows are intact until phase 3
+    phase_saves<NP, COMMIT, NW, VerifySmem<NP>, VerifySmem<NP>, CS>(P, it, tid, sm, sm, col0);
   if constexpr (!kHalves) {
     bf16x8 wh[NP / 32][TT], wl[NP / 32][TT];
     phase_w<NP, NWC>(lane, wave, sm, sm, ck, wh, wl, col0);
@@ -2516,7 +2539,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& P, int tid_in, i
     phase_stores<NP, COMMIT, NW, VerifySmem<NP>, CS>(P, it, tid_s, sm, col0);
   }
   if constexpr (COMMIT)
-    if (it.h == 0 && wave == 0) fused_status(it, lane, sm.graw[4][lane & 15], sm.graw[4]);
+    if (it.h == 0 && wave == 0 && col0 == 0) fused_status(it, lane, sm.graw[4][lane & 15], sm.graw[4]);
 }
 
 // Both widths run at 4 waves per SIMD (at most 128 registers): the 32-wide
@@ -2594,10 +2617,10 @@ static_assert(std::is_trivially_copyable<VerifyParams>::value, "VerifyParams is 
 // RAWK: the pending keys are the previous step's raw bf16 rows; RVN: the
 // path's values are recomputed from raw rows; PDMA: (32-wide, both raw)
 // those rows are copied into LDS ahead of the state tile
-template <int NP, bool RAWK, bool RVN, bool PDMA = false>
+template <int NP, bool RAWK, bool RVN, bool PDMA = false, int CS = 1>
 __global__ void __launch_bounds__(64 * WavesFor<NP>()) __attribute__((amdgpu_waves_per_eu(4)))
 tree_commit_verify_kernel(const VerifyParams P) {
-  verify_body<NP, true, true, RAWK, RVN, PDMA>(P, threadIdx.x, blockIdx.x, Given{});
+  verify_body<NP, true, true, RAWK, RVN, PDMA, CS>(P, threadIdx.x, blockIdx.x, Given{});
 }
 
 static VerifyParams make_params(const dft_verify_args* a) {
@@ -2700,7 +2723,15 @@ int launch_size_order(const int32_t* cu_seqlens, int batch, int n_nodes, int32_t
 // Launches over 32 nodes with at most kSplitItems64 items do the same with
 // the 64-wide kernel (tail_halves; 110 KiB of LDS, one workgroup per CU, so
 // at most 256 workgroups for the 256 CUs).
-constexpr int kSplitItems = 256, kSplitItems64 = 128;
+// The fused commit -> verify of up to 32 nodes splits its columns the same
+// way up to kSplitItemsFused items (three of its workgroups fit a CU, by LDS
+// and registers: 768 in one generation).  24 layers: batch 1 (32 items) 367
+// -> 297 us, batch 4 (27 nodes) 414 -> 341, batch 8 432 -> 407, batch 12 530
+// -> 512; batch 16 (512 items) would go from 545 to 763.  The split halves
+// hold half the tile's registers, which also makes room for the whole-wave
+// diagonal solves (367 -> 348 us at batch 4), and take their v rows with the
+// q/k rows instead of behind the write-back.
+constexpr int kSplitItems = 256, kSplitItems64 = 128, kSplitItemsFused = 384;
 
 int launch_tree_verify(const dft_verify_args* a, hipStream_t stream) {
   const VerifyParams P = make_params(a);
@@ -2757,19 +2788,25 @@ int launch_tree_commit_verify(const dft_verify_args* a, const dft_pending_commit
   const auto al16 = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
   const bool pdma = form == 3 && al16(c->key_rows) && al16(c->value_rows) && c->kr_h_stride % 8 == 0 &&
                     c->kr_row_stride % 8 == 0 && c->vr_h_stride % 8 == 0 && c->vr_row_stride % 8 == 0;
-#define DFT_FUSED(np, g, b, prm)                                                                               \
-  switch (form) {                                                                                              \
-    case 0: hipLaunchKernelGGL((tree_commit_verify_kernel<np, false, false>), g, b, 0, stream, prm); break;   \
-    case 1: hipLaunchKernelGGL((tree_commit_verify_kernel<np, true, false>), g, b, 0, stream, prm); break;    \
-    case 2: hipLaunchKernelGGL((tree_commit_verify_kernel<np, false, true>), g, b, 0, stream, prm); break;    \
-    default: hipLaunchKernelGGL((tree_commit_verify_kernel<np, true, true>), g, b, 0, stream, prm); break;    \
+  const int64_t items = (int64_t)a->batch * a->hv;
+  const dim3 grid2((unsigned)(2 * items));
+#define DFT_FUSED(np, cs, g, b, prm)                                                                                   \
+  switch (form) {                                                                                                      \
+    case 0: hipLaunchKernelGGL((tree_commit_verify_kernel<np, false, false, false, cs>), g, b, 0, stream, prm); break; \
+    case 1: hipLaunchKernelGGL((tree_commit_verify_kernel<np, true, false, false, cs>), g, b, 0, stream, prm); break;  \
+    case 2: hipLaunchKernelGGL((tree_commit_verify_kernel<np, false, true, false, cs>), g, b, 0, stream, prm); break;  \
+    default: hipLaunchKernelGGL((tree_commit_verify_kernel<np, true, true, false, cs>), g, b, 0, stream, prm); break;  \
   }
-  if (a->n_nodes > 32) DFT_FUSED(64, grid, block64, wide)
+  if (a->n_nodes > 32) DFT_FUSED(64, 1, grid, block64, wide)
   if (a->n_nodes <= 32 || split) {
-    if (pdma)
+    if (pdma && items <= kSplitItemsFused)
+      hipLaunchKernelGGL((tree_commit_verify_kernel<32, true, true, true, 2>), grid2, block, 0, stream, narrow);
+    else if (pdma)
       hipLaunchKernelGGL((tree_commit_verify_kernel<32, true, true, true>), grid, block, 0, stream, narrow);
+    else if (items <= kSplitItemsFused)
+      DFT_FUSED(32, 2, grid2, block, narrow)
     else
-      DFT_FUSED(32, grid, block, narrow)
+      DFT_FUSED(32, 1, grid, block, narrow)
   }
 #undef DFT_FUSED
   return hipGetLastError() == hipSuccess ? DFT_OK : DFT_ERR_LAUNCH;

@@ -498,3 +498,63 @@ def test_commit_verify_many_items_chain_of_three(cuda):
     got = np32(pool)
     for r in range(B):
         assert rel_l2(got[r].transpose(0, 2, 1), S[r]) <= REL_L2, r
+
+
+@pytest.mark.parametrize("raw_keys,raw_values,pad", [(False, False, 0), (True, False, 0), (False, True, 0),
+                                                     (True, True, 0), (True, True, 4)])
+@pytest.mark.parametrize("N", [5, 17, 32])
+def test_commit_verify_column_split(cuda, raw_keys, raw_values, pad, N):
+    """A launch whose items take one workgroup each (13 requests of 32 heads)
+    against the same requests in launches that split every item's columns
+    over two (7 and 6, then one by one): the same bits in o, the saves, the
+    committed states and the status words, for every form of the pending
+    path, with an empty path and a request without a slot."""
+    from dforktree_amd import ops, synth
+    announce(f"commit->verify column split N={N} raw keys {raw_keys} values {raw_values} pad {pad}")
+    B, hk, hv = 13, 16, 32
+    b1 = synth.make_batch(80, 0, [N] * B, hk=hk, hv=hv)
+    b2 = synth.make_batch(81, 0, [N] * B, hk=hk, hv=hv)
+    g1, g2 = b1.to(cuda), b2.to(cuda)
+    rows = B * N
+    k1 = torch.zeros(hk, rows, 128, device=cuda)
+    v1 = torch.zeros(hv, rows, 128, device=cuda)
+    G1 = torch.zeros(hv, rows, device=cuda)
+    pool0 = b1.state.clone().to(cuda)
+    ts1 = ops.tree_struct(g1.parent, 4, batch=B, n_nodes=N, want=("anc_bits",))["anc_bits"]
+    ts2 = ops.tree_struct(g2.parent, 4, batch=B, n_nodes=N, want=("anc_bits",))["anc_bits"]
+    ops.tree_verify(g1.y, g1.a, g1.b, g1.A_log, g1.dt_bias, pool0.transpose(-1, -2), hk=hk, hv=hv, anc_bits=ts1,
+                    batch=B, n_nodes=N, aux_k=k1, aux_v=v1, aux_g=G1, aux_k_per_khead=True)
+    idx, lens, _ = _paths(b1, 82, empty=(3,))
+    idx, lens = idx.to(cuda), lens.to(cuda)
+    slots = torch.arange(B, dtype=torch.int32, device=cuda)
+    slots[5] = -1
+    slots[0] = 5  # (slot 0, which the slotless request reads, is no one's)
+    y1 = g1.y
+    if pad:
+        y1 = torch.empty(rows, y1.shape[1] + pad, dtype=y1.dtype, device=cuda)[:, :y1.shape[1]]
+        y1.copy_(g1.y)
+
+    def run(cuts):
+        pool, status = pool0.clone(), torch.full((B,), -1, dtype=torch.int32, device=cuda)
+        o = torch.zeros(rows, hv, 128, dtype=torch.bfloat16, device=cuda)
+        aux = (torch.zeros_like(k1), torch.zeros_like(v1), torch.zeros_like(G1))
+        for lo, hi in zip(cuts[:-1], cuts[1:]):
+            sl = slice(lo * N, hi * N)
+            kw = (dict(pending_keys=None, pending_key_rows=y1[sl, hk * 128:2 * hk * 128].unflatten(1, (hk, 128)))
+                  if raw_keys else dict(pending_keys=k1[:, sl]))
+            kw.update(dict(pending_values=None, pending_value_rows=y1[sl, 2 * hk * 128:].unflatten(1, (hv, 128)),
+                           pending_b=g1.b[sl]) if raw_values else dict(pending_values=v1[:, sl]))
+            ops.tree_commit_verify(g2.y[sl], g2.a[sl], g2.b[sl], g2.A_log, g2.dt_bias, pool.transpose(-1, -2), hk=hk,
+                                   hv=hv, anc_bits=ts2[sl], batch=hi - lo, n_nodes=N, state_indices=slots[lo:hi],
+                                   o=o[sl], aux_k=aux[0][:, sl], aux_v=aux[1][:, sl], aux_g=aux[2][:, sl],
+                                   aux_k_per_khead=True, status=status[lo:hi], pending_path=idx[lo:hi],
+                                   pending_path_len=lens[lo:hi], pending_gains=G1[:, sl], prev_n_nodes=N,
+                                   pending_k_head_div=hv // hk, pending_anc_bits=ts1[sl], **kw)
+        torch.cuda.synchronize()
+        return (pool, o, *aux, status)
+
+    whole = run([0, B])
+    assert not torch.equal(whole[0], pool0)
+    for cuts in ([0, 7, B], list(range(B + 1))):
+        for x, y in zip(whole, run(cuts)):
+            assert torch.equal(x, y)
