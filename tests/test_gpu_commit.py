@@ -286,3 +286,56 @@ def test_config4_full_size_verify_then_commit_matches_replay(cuda):
                                  before[(l, b)].transpose(0, 2, 1), path, HK, HV, D, D)
         err = rel_l2(np32(S[l, b]).transpose(0, 2, 1), want)
         assert err <= REL_L2, (l, b, len(path), err)
+
+
+# path lengths around a wave's pairs of row copies (2, 8, 10, 16) and up to a
+# whole 64-node path, gaps in the path, both layouts, aligned rows and not,
+# int32 and int64 indices; the state, the destination and the other slots
+@pytest.mark.parametrize("cols,lens", [(1, (1,)), (2, (0, 2)), (7, (3, 7)), (16, (8, 9, 10, 16)), (17, (15, 17)),
+                                       (64, (31, 63, 64))])
+@pytest.mark.parametrize("aligned", [True, False])
+@pytest.mark.parametrize("kv_layout", [False, True])
+def test_commit_path_lengths(cuda, cols, lens, aligned, kv_layout):
+    from dforktree_amd import ops
+    announce(f"commit path lengths cols={cols} lens={lens} aligned={aligned} kv={kv_layout}")
+    L, B, H, HK, N = 2, len(lens), 4, 2, 64
+    g = torch.Generator().manual_seed(cols)
+    off = 0 if aligned else 1
+    S = torch.randn(L, B + 2, H, 128, 128, generator=g) * 0.1
+    k = torch.nn.functional.normalize(torch.randn(L, HK, B * N, 128, generator=g), dim=-1)
+    v = torch.randn(L, H, B * N, 128, generator=g)
+    G = -torch.rand(L, H, B * N, generator=g) * 3
+    path = torch.full((B, cols), -1, dtype=torch.int64)
+    for b, n in enumerate(lens):
+        path[b, :n] = torch.randperm(N, generator=g)[:n]
+        if n > 4:
+            path[b, 2] = -1       # a gap
+            path[b, n - 2] = 999  # past the tree: ignored
+    slots = torch.randperm(B + 2, generator=g)[:B]
+
+    def dev(t, pad=off):
+        buf = torch.zeros(t.numel() + 8, device=cuda)
+        buf[pad:pad + t.numel()] = t.reshape(-1).to(cuda)
+        return buf[pad:pad + t.numel()].view(t.shape)
+    for it in (torch.int32, torch.int64):
+        Sd = dev(S, 0)
+        ops.tree_commit(Sd, dev(k), dev(v), G.to(cuda), path.to(it).to(cuda), n_nodes=N, src_slots=slots.to(it).to(cuda),
+                        kv_layout=kv_layout, k_head_div=H // HK)
+        got = Sd.cpu().double()
+        want = S.double().clone()
+        for b in range(B):
+            ok = [int(x) for x in path[b] if 0 <= x < N]
+            if not ok:
+                continue
+            rows = [b * N + t for t in ok]
+            Gb = G.double()[:, :, rows]
+            w = (Gb[:, :, -1:] - Gb).exp()
+            kk = k.double()[:, :, rows].repeat_interleave(H // HK, 1)
+            up = torch.matmul((v.double()[:, :, rows] * w[..., None]).transpose(-1, -2).contiguous(), kk)  # [L, H, V, K]
+            if kv_layout:
+                up = up.transpose(-1, -2)
+            want[:, slots[b]] = Gb[:, :, -1].exp()[..., None, None] * S.double()[:, slots[b]] + up
+        # fp32 sums of at most 64 products of order 1, weights of 1e-6 relative
+        assert float((got - want).abs().max()) <= 64 * 4e-6
+        untouched = [s for s in range(B + 2) if s not in slots.tolist()]
+        assert torch.equal(Sd.cpu()[:, untouched], S[:, untouched])
