@@ -2000,6 +2000,14 @@ struct Given {
   int lds_off;
 };
 
+// The same of the fused kernel (tree_commit_verify_mixed_kernel), whose items
+// also hold the recomputed path values' matrices and norms.
+template <int NP>
+constexpr int kFusedItemLds = sizeof(VerifySmem<NP>) + kRvx * sizeof(float);
+constexpr int kMixedFusedLds = kFusedItemLds<64> > 2 * kFusedItemLds<32> ? kFusedItemLds<64> : 2 * kFusedItemLds<32>;
+static_assert(kFusedItemLds<32> % 16 == 0 && kMixedFusedLds <= 80 * 1024, "two mixed fused workgroups per CU");
+__shared__ uint4 mixed_fused_lds[kMixedFusedLds / 16];
+
 // k-step s (rows k = 32s .. 32s + 31) of column tile c's state, in the MFMA layout
 __device__ __forceinline__ void issue_state_half(const float* S0, int64_t v_stride, int c, int lane, int s,
                                                  f32x4& a, f32x4& b) {
@@ -2243,11 +2251,12 @@ __device__ __forceinline__ void verify_body(const VerifyParams& P, int tid_in, i
   constexpr int kQkvDma = kPlanes * (NP / (4 * NW));          // row copies per wave
   constexpr int kStateLoads = 8 * TT, kGroupLoads = 2 * TT;   // per lane: whole tile, one k-step group
   const dft_verify_args& p = P.a;
-  static_assert(!GIVEN || (!COMMIT && CS == 1), "a given item is a plain verify");
-  // the verify's arrays: the body's own, or (a given item) its region of mixed_lds
+  static_assert(!GIVEN || CS == 1, "a given item takes one workgroup or half of one");
+  // the verify's arrays: the body's own, or (a given item) its region of the mixed kernel's
   VerifySmem<NP>& sm = [&]() -> VerifySmem<NP>& {
     if constexpr (GIVEN) {
-      return *reinterpret_cast<VerifySmem<NP>*>(reinterpret_cast<char*>(mixed_lds) + given.lds_off);
+      return *reinterpret_cast<VerifySmem<NP>*>(reinterpret_cast<char*>(COMMIT ? mixed_fused_lds : mixed_lds) +
+                                                given.lds_off);
     } else {
       __shared__ VerifySmem<NP> own;
       return own;
@@ -2257,7 +2266,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& P, int tid_in, i
   // recompute them hold them (4.3 KiB)
   float* const rvx = [&]() -> float* {
     if constexpr (GIVEN) {
-      return nullptr;
+      return reinterpret_cast<float*>(&sm + 1);
     } else {
       __shared__ alignas(16) float own[RVN ? kRvx : 4];
       return own;
@@ -2552,32 +2561,34 @@ __global__ void __launch_bounds__(64 * WavesFor<NP>())
   verify_body<NP, S0VEC, false, false, false, false, CS>(P, threadIdx.x, blockIdx.x, Given{});
 }
 
-// A packed batch with trees on both sides of 32 nodes and size-order records,
-// in one launch of 8-wave workgroups (2 per CU: the LDS of one 64-wide item
-// or of two 32-wide ones).  Blocks [0, c1 Hv) take the (request, v-head)
+// A packed batch with trees on both sides of 32 nodes in one launch of 8-wave
+// workgroups (2 per CU: the LDS of one 64-wide item or of two 32-wide ones).
+// With size-order records, blocks [0, c1 Hv) take the (request, v-head)
 // items of the c1 requests over 32 nodes on the 64-wide body; each block
 // after them takes v-heads 2j and 2j + 1 of one of the c0 other requests,
 // one per half of the workgroup (4 waves each) on the 32-wide body.  The two
-// halves verify the same tree (same node count, same exits), so they pass the
-// same barriers.  The 64-wide class's last generation then shares the chip
-// with the small trees instead of leaving most of it idle in front of a
-// second kernel.
-// Records of another launch shape are ignored: block b then takes item b
-// and its request's size picks the body; a small tree's v-heads 2j, 2j + 1
-// go to the block of head 2j, and the other block exits.  Either way every
-// item runs the body of its size class, as in the two-kernel launch.
-template <bool S0VEC>
-__global__ void __launch_bounds__(64 * WavesFor<64>()) __attribute__((amdgpu_waves_per_eu(4)))
-tree_verify_mixed_kernel(const VerifyParams P) {
+// halves verify the same tree (same node count, same path, same exits), so
+// they pass the same barriers.  The 64-wide class's last generation then
+// shares the chip with the small trees instead of leaving most of it idle in
+// front of a second kernel.
+// Without records, or with those of another launch shape (ignored), block b
+// takes item b and its request's size picks the body; a small tree's v-heads
+// 2j, 2j + 1 go to the block of head 2j, and the other block exits.  Either
+// way every item runs the body of its size class, as in the two-kernel
+// launch, with the same bits.
+
+// Where block `blockIdx.x` of a mixed launch finds its work: returns false if
+// it has none; `wide`: one 64-wide item, else two 32-wide ones (g: that of
+// this thread's half).
+__device__ __forceinline__ bool mixed_item(const VerifyParams& P, Given& g, bool& wide, int lds32) {
   const dft_verify_args& p = P.a;
-  const int4 hd = reinterpret_cast<const int4*>(p.size_order)[0];
-  const bool rec = hd.z == p.n_nodes && hd.w == p.batch;  // uniform
+  int4 hd = make_int4(0, 0, 0, 0);
+  if (p.size_order) hd = reinterpret_cast<const int4*>(p.size_order)[0];
+  const bool rec = p.size_order && hd.z == p.n_nodes && hd.w == p.batch;  // uniform
   const int blk = blockIdx.x, half = threadIdx.x >> 8, R = p.hv / p.hk;
-  Given g;
   g.n_lo = INT_MIN;
   g.n_hi = INT_MAX;
   g.lds_off = 0;
-  bool wide;
   if (rec) {
     const int c0 = hd.x, c1 = hd.y, hp = p.hv >> 1;
     wide = blk < c1 * p.hv;
@@ -2586,7 +2597,7 @@ tree_verify_mixed_kernel(const VerifyParams P) {
       g.cls = 1;
     } else {
       const int j = blk - c1 * p.hv;
-      if (j >= c0 * hp) return;
+      if (j >= c0 * hp) return false;
       g.it.b = j / hp;
       g.it.h = 2 * (j - g.it.b * hp);
       g.cls = 0;
@@ -2595,20 +2606,30 @@ tree_verify_mixed_kernel(const VerifyParams P) {
     item_heads(p, blk, g.it);
     const int span = p.cu_seqlens[g.it.b + 1] - p.cu_seqlens[g.it.b];
     wide = span > 32;  // (cut to n_nodes, which is over 32 here)
-    if (!wide && (g.it.h & 1)) return;
+    if (!wide && (g.it.h & 1)) return false;
     g.cls = -1;
     if (wide) g.n_lo = 33;
   }
-  if (wide) {
-    verify_body<64, S0VEC, false, false, false, false, 1, true>(P, threadIdx.x, blk, g);
-  } else {
+  if (!wide) {
     g.it.h += half;
     g.it.hk = g.it.h / R;
     g.it.rr = g.it.h - g.it.hk * R;
     g.n_hi = 32;
-    g.lds_off = half * (int)sizeof(VerifySmem<32>);
-    verify_body<32, S0VEC, false, false, false, false, 1, true>(P, threadIdx.x & 255, blk, g);
+    g.lds_off = half * lds32;
   }
+  return true;
+}
+
+template <bool S0VEC>
+__global__ void __launch_bounds__(64 * WavesFor<64>()) __attribute__((amdgpu_waves_per_eu(4)))
+tree_verify_mixed_kernel(const VerifyParams P) {
+  Given g;
+  bool wide;
+  if (!mixed_item(P, g, wide, (int)sizeof(VerifySmem<32>))) return;
+  if (wide)
+    verify_body<64, S0VEC, false, false, false, false, 1, true>(P, threadIdx.x, blockIdx.x, g);
+  else
+    verify_body<32, S0VEC, false, false, false, false, 1, true>(P, threadIdx.x & 255, blockIdx.x, g);
 }
 
 // P must stay this kernel's first (only) argument: out_args<true> reads it
@@ -2621,6 +2642,20 @@ template <int NP, bool RAWK, bool RVN, bool PDMA = false, int CS = 1>
 __global__ void __launch_bounds__(64 * WavesFor<NP>()) __attribute__((amdgpu_waves_per_eu(4)))
 tree_commit_verify_kernel(const VerifyParams P) {
   verify_body<NP, true, true, RAWK, RVN, PDMA, CS>(P, threadIdx.x, blockIdx.x, Given{});
+}
+
+// The mixed-width launch of the fused commit -> verify (PDMA: of its 32-wide
+// items).  The two halves of a workgroup commit the same request's path.
+template <bool RAWK, bool RVN, bool PDMA>
+__global__ void __launch_bounds__(64 * WavesFor<64>()) __attribute__((amdgpu_waves_per_eu(4)))
+tree_commit_verify_mixed_kernel(const VerifyParams P) {
+  Given g;
+  bool wide;
+  if (!mixed_item(P, g, wide, kFusedItemLds<32>)) return;
+  if (wide)
+    verify_body<64, true, true, RAWK, RVN, false, 1, true>(P, threadIdx.x, blockIdx.x, g);
+  else
+    verify_body<32, true, true, RAWK, RVN, PDMA, 1, true>(P, threadIdx.x & 255, blockIdx.x, g);
 }
 
 static VerifyParams make_params(const dft_verify_args* a) {
@@ -2649,10 +2684,10 @@ static VerifyParams make_params(const dft_verify_args* a) {
 // The 64-wide kernel goes first: the reverse order measured 0.4% slower on
 // 128 requests of 8-64 nodes.  With size-order records each kernel takes its
 // own class's requests from the front of its grid, and its exiting blocks
-// come last.  The plain verify with records, a vector state and an even
-// v-head count runs instead as the one mixed-width kernel
-// (tree_verify_mixed_kernel): 112.98 -> 111.65 and 112.12 -> 110.28 us per
-// ragged layer in interleaved runs on two boxes.
+// come last.  With a vector state and an even v-head count most such launches
+// run instead as one mixed-width kernel (mixed_launch): the verify of 128
+// requests of 8-64 nodes 112.98 -> 111.65 and 112.12 -> 110.28 us per layer in
+// interleaved runs on two boxes.
 static void split_by_size(const dft_verify_args* a, const VerifyParams& P, VerifyParams& narrow, VerifyParams& wide,
                           bool& split) {
   narrow = wide = P;
@@ -2715,6 +2750,22 @@ int launch_size_order(const int32_t* cu_seqlens, int batch, int n_nodes, int32_t
   return hipGetLastError() == hipSuccess ? DFT_OK : DFT_ERR_LAUNCH;
 }
 
+// Whether a launch split by tree size runs as one mixed-width launch: with
+// size-order records, and without them in small launches, where the second
+// kernel's start and the emptier chip cost more than the workgroups that
+// exit between the others.  us per 8 layers of 8-64 nodes, 32 heads, two
+// kernels / one:
+//   verify + commit, records     batch 2 174 / 128, 8 170 / 163, 32 428 / 418
+//   fused (raw rows), records    batch 2 234 / 150, 8 277 / 170, 48 562 / 531
+//   fused (saves), records       batch 16 291 / 241, 32 415 / 372, 48 611 / 542
+//   fused (raw rows), none       batch 2 232 / 150, 24 401 / 379, 48 619 / 668
+//   fused (saves), none          batch 16 349 / 243, 32 469 / 451, 48 621 / 649
+// (the forms other than raw rows spill 6-8 registers in the mixed kernel).
+constexpr int64_t kMixedItems = 768;
+static bool mixed_launch(const dft_verify_args* a, bool split) {
+  return split && a->hv % 2 == 0 && (a->size_order || (int64_t)a->batch * a->hv <= kMixedItems);
+}
+
 // Launches of up to 32 nodes whose items would leave most of the chip idle
 // (at most kSplitItems of them: batch 1 at 32 v-heads is 32) split each
 // item's value columns over two workgroups: each forms phase 1 in full and
@@ -2740,6 +2791,10 @@ int launch_tree_verify(const dft_verify_args* a, hipStream_t stream) {
   bool split;
   split_by_size(a, P, narrow, wide, split);
   const int64_t items = (int64_t)a->batch * a->hv;
+  if (P.s0_vec && mixed_launch(a, split)) {
+    hipLaunchKernelGGL((tree_verify_mixed_kernel<true>), grid, block64, 0, stream, P);
+    return hipGetLastError() == hipSuccess ? DFT_OK : DFT_ERR_LAUNCH;
+  }
   if (a->n_nodes > 32 && items <= kSplitItems64 && P.s0_vec) {
     const dim3 grid2((unsigned)(2 * items));
     hipLaunchKernelGGL((tree_verify_kernel<64, true, 2>), grid2, block64, 0, stream, wide);
@@ -2752,10 +2807,6 @@ int launch_tree_verify(const dft_verify_args* a, hipStream_t stream) {
       hipLaunchKernelGGL((tree_verify_kernel<32, true, 2>), grid2, block, 0, stream, narrow);
     else
       hipLaunchKernelGGL((tree_verify_kernel<32, false, 2>), grid2, block, 0, stream, narrow);
-    return hipGetLastError() == hipSuccess ? DFT_OK : DFT_ERR_LAUNCH;
-  }
-  if (split && a->size_order && P.s0_vec && a->hv % 2 == 0) {
-    hipLaunchKernelGGL((tree_verify_mixed_kernel<true>), grid, block64, 0, stream, P);
     return hipGetLastError() == hipSuccess ? DFT_OK : DFT_ERR_LAUNCH;
   }
   if (a->n_nodes > 32) {
@@ -2796,6 +2847,17 @@ int launch_tree_commit_verify(const dft_verify_args* a, const dft_pending_commit
     case 1: hipLaunchKernelGGL((tree_commit_verify_kernel<np, true, false, false, cs>), g, b, 0, stream, prm); break;  \
     case 2: hipLaunchKernelGGL((tree_commit_verify_kernel<np, false, true, false, cs>), g, b, 0, stream, prm); break;  \
     default: hipLaunchKernelGGL((tree_commit_verify_kernel<np, true, true, false, cs>), g, b, 0, stream, prm); break;  \
+  }
+  if (mixed_launch(a, split)) {
+    if (pdma)
+      hipLaunchKernelGGL((tree_commit_verify_mixed_kernel<true, true, true>), grid, block64, 0, stream, P);
+    else switch (form) {
+      case 0: hipLaunchKernelGGL((tree_commit_verify_mixed_kernel<false, false, false>), grid, block64, 0, stream, P); break;
+      case 1: hipLaunchKernelGGL((tree_commit_verify_mixed_kernel<true, false, false>), grid, block64, 0, stream, P); break;
+      case 2: hipLaunchKernelGGL((tree_commit_verify_mixed_kernel<false, true, false>), grid, block64, 0, stream, P); break;
+      default: hipLaunchKernelGGL((tree_commit_verify_mixed_kernel<true, true, false>), grid, block64, 0, stream, P); break;
+    }
+    return hipGetLastError() == hipSuccess ? DFT_OK : DFT_ERR_LAUNCH;
   }
   if (a->n_nodes > 32) DFT_FUSED(64, 1, grid, block64, wide)
   if (a->n_nodes <= 32 || split) {

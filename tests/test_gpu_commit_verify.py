@@ -558,3 +558,74 @@ def test_commit_verify_column_split(cuda, raw_keys, raw_values, pad, N):
     for cuts in ([0, 7, B], list(range(B + 1))):
         for x, y in zip(whole, run(cuts)):
             assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("raw_keys,raw_values,pad", [(False, False, 0), (True, False, 0), (False, True, 0),
+                                                     (True, True, 0), (True, True, 4)])
+def test_commit_verify_mixed_kernel(cuda, raw_keys, raw_values, pad):
+    """A packed batch on both sides of 32 nodes, with empty trees, an empty
+    path and a request without a slot: as one mixed-width launch with
+    size-order records, as two kernels without them (26 requests of 32 heads
+    are past the record-less limit), and as two record-less mixed launches of
+    13 requests: the same bits in every output."""
+    from dforktree_amd import ops, synth
+    announce(f"commit->verify mixed kernel raw keys {raw_keys} values {raw_values} pad {pad}")
+    hk, hv = 16, 32
+    sizes = [[40, 9, 0, 64, 17, 33, 1, 32, 48, 5, 16, 63, 20], [31, 34, 2, 60, 0, 12, 33, 50, 8, 64, 25, 3, 49]]
+    prev = [[7, 64, 33, 0, 20, 32, 41, 1, 16, 30, 63, 5, 48], [33, 2, 18, 64, 32, 0, 40, 9, 31, 50, 4, 36, 12]]
+    flat, pflat = sum(sizes, []), sum(prev, [])
+    B = len(flat)
+    g = torch.Generator().manual_seed(7)
+
+    def trees(ns):
+        cu = torch.tensor(np.concatenate([[0], np.cumsum(ns)]), dtype=torch.int32)
+        par = torch.cat([synth.tree_parents(n, "random", g) for n in ns if n])
+        bits = ops.tree_struct(par.to(cuda), 4, cu_seqlens=cu.to(cuda), n_nodes=64, batch=B, want=("anc_bits",))
+        return cu, par, bits["anc_bits"]
+    cu, _, bits = trees(flat)
+    pcu, ppar, pbits = trees(pflat)
+    C = (2 * hk + hv) * 128
+    rows, prows = int(cu[-1]), int(pcu[-1])
+
+    def rand(*shape, std=1.0, dtype=torch.bfloat16):
+        return (torch.randn(*shape, generator=g) * std).to(dtype).to(cuda)
+    y, a, b = rand(rows, C), rand(rows, hv), rand(rows, hv)
+    py, pb = rand(prows, C + pad)[:, :C], rand(prows, hv)
+    A_log, dtb = rand(hv, std=0.3, dtype=torch.float32), rand(hv, std=0.3, dtype=torch.float32)
+    pool0 = rand(B, hv, 128, 128, std=0.02, dtype=torch.float32)
+    pk = torch.nn.functional.normalize(rand(hk, prows, 128, dtype=torch.float32), dim=-1)
+    pv, pG = rand(hv, prows, 128, std=0.3, dtype=torch.float32), -rand(hv, prows, dtype=torch.float32).abs()
+    path = torch.full((B, 16), -1, dtype=torch.int32)
+    for r, n in enumerate(pflat):
+        if n and r != 4:
+            walk = synth.accepted_path(ppar[int(pcu[r]):int(pcu[r + 1])], 16, g)
+            path[r, :len(walk)] = walk
+    slots = torch.arange(B, dtype=torch.int32)
+    slots[5], slots[0] = -1, 5  # (slot 0, which the slotless request reads, is no one's)
+    path, slots = path.to(cuda), slots.to(cuda)
+
+    def run(cuts, records):
+        pool = pool0.clone()
+        o = torch.zeros(rows, hv, 128, dtype=torch.bfloat16, device=cuda)
+        k, v, G = (torch.zeros(h, rows, *t, device=cuda) for h, t in ((hk, (128,)), (hv, (128,)), (hv, ())))
+        status = torch.full((B,), -1, dtype=torch.int32, device=cuda)
+        for lo, hi in zip(cuts[:-1], cuts[1:]):
+            cd, pcd = cu[lo:hi + 1].to(cuda), pcu[lo:hi + 1].to(cuda)  # (absolute rows: the buffers are whole)
+            kw = (dict(pending_keys=None, pending_key_rows=py[:, hk * 128:2 * hk * 128].unflatten(1, (hk, 128)))
+                  if raw_keys else dict(pending_keys=pk))
+            kw.update(dict(pending_values=None, pending_value_rows=py[:, 2 * hk * 128:].unflatten(1, (hv, 128)),
+                           pending_b=pb) if raw_values else dict(pending_values=pv))
+            ops.tree_commit_verify(y, a, b, A_log, dtb, pool.transpose(-1, -2), hk=hk, hv=hv, anc_bits=bits,
+                                   batch=hi - lo, n_nodes=64, cu_seqlens=cd, state_indices=slots[lo:hi], o=o, aux_k=k,
+                                   aux_v=v, aux_g=G, aux_k_per_khead=True, status=status[lo:hi],
+                                   size_order=ops.size_order(cd, 64) if records else None, pending_path=path[lo:hi],
+                                   pending_gains=pG, prev_cu_seqlens=pcd, pending_k_head_div=hv // hk,
+                                   pending_anc_bits=pbits, **kw)
+        torch.cuda.synchronize()
+        return pool, o, k, v, G, status
+
+    two = run([0, B], False)
+    assert not torch.equal(two[0], pool0) and bool((two[5] == 0).all())
+    for other in (run([0, B], True), run([0, 13, B], False)):
+        for x, z in zip(two, other):
+            assert torch.equal(x, z)
