@@ -236,13 +236,26 @@ __global__ void __launch_bounds__(64) tree_conv4_bf16_kernel(const dft_conv_args
 // 54.8 us per launch with a one-wave workgroup per node that gathered its
 // four rows from memory, 37.2 here, 4.5 TB/s; a streaming probe moves 5.2
 // TB/s at this mix of reads and writes.  The same rows in cache: 42.0 -> 32.8.
-// Batch 4: 8.2 -> 5.6, batch 1 (plugin step, 24 layers): 354 -> 334.  4 waves
-// took 1.2 us longer, 16 4 us.
+// Batch 4: 8.2 -> 5.6, batch 1 (plugin step, 24 layers): 354 -> 334, and 330
+// -> 318 once no load of the prologue waited for another.  4 waves took 1.2 us
+// longer, 16 4 us.
 constexpr int kConvNodes = 64, kConvSlice = 256, kConvWaves = 8;
 
 // rows of the workgroup's LDS: zeros, 3 state columns, the tokens (an odd
 // count's last copy fills one more)
 __host__ __device__ constexpr int conv_rows(int n) { return 4 + n + (n & 1); }
+
+// Request b's index (b itself without an array) by scalar loads: the array is
+// not written by the launch.
+__device__ __forceinline__ int64_t uniform_req_index(const void* idx, int dt, int b) {
+  if (!idx) return b;
+  typedef const __attribute__((address_space(4))) int32_t* Words;
+  const Words w = (Words)(uintptr_t)idx;
+  const bool wide = dt == DFT_I64;
+  const int half = wide ? 0 : 1;  // (shifts: selected addresses become a branch)
+  const int32_t lo = w[(2 * b) >> half], hi = w[(2 * b + 1) >> half];
+  return wide ? (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo) : (int64_t)lo;
+}
 
 // 4 channels (of lane l) of the four rows at these byte offsets
 __device__ __forceinline__ void tap_rows(const uint16_t* rows, const int* taps, int n, int lane, uint2 (&r)[4]) {
@@ -257,6 +270,15 @@ __device__ __forceinline__ void tap_rows(const uint16_t* rows, const int* taps, 
 template <bool CIDX64>
 __global__ void __launch_bounds__(64 * kConvWaves) tree_conv4_rows_kernel(const dft_conv_args p, int cblocks,
                                                                           int splits) {
+  // Every load of the prologue goes out before anything waits for one of
+  // them: read where they are used, the tap columns were waited for (and with
+  // them the row copies ahead of them) before the weights and the state were
+  // asked for.  The arguments are forced into scalar registers first, for the
+  // same reason.
+  asm volatile("" ::"s"(p.batch), "s"(p.n_nodes), "s"(p.channels), "s"(p.x), "s"(p.x_req_stride), "s"(p.x_node_stride), "s"(p.conv_state), "s"(p.cs_slot_stride),
+               "s"(p.cs_chan_stride), "s"(p.cs_col_stride), "s"(p.cs_indices), "s"(p.cs_indices_dtype), "s"(p.weight),
+               "s"(p.cidx), "s"(p.cidx_req_stride), "s"(p.cidx_node_stride), "s"(p.iw_indices), "s"(p.iw_indices_dtype),
+               "s"(cblocks), "s"(splits));
   extern __shared__ u32x4 conv_lds[];
   const int N = p.n_nodes;
   uint16_t* rows = reinterpret_cast<uint16_t*>(conv_lds);                // [conv_rows(N)][256]
@@ -272,8 +294,8 @@ __global__ void __launch_bounds__(64 * kConvWaves) tree_conv4_rows_kernel(const 
   const int cbase = cb * kConvSlice, nch = min(kConvSlice, p.channels - cbase);  // a multiple of 8
 
   // the slots (a negative state slot reads slot 0, a negative window slot writes no window)
-  const int64_t slot_raw = p.cs_indices ? req_index(p.cs_indices, p.cs_indices_dtype, b) : b;
-  const int64_t dst = p.iw_indices ? req_index(p.iw_indices, p.iw_indices_dtype, b) : b;
+  const int64_t slot_raw = uniform_req_index(p.cs_indices, p.cs_indices_dtype, b);
+  const int64_t dst = uniform_req_index(p.iw_indices, p.iw_indices_dtype, b);
   {
     // (channels past the last read channel 0 of the slice instead)
     const uint16_t* xb = static_cast<const uint16_t*>(p.x) + (int64_t)b * p.x_req_stride + cbase;
@@ -282,40 +304,43 @@ __global__ void __launch_bounds__(64 * kConvWaves) tree_conv4_rows_kernel(const 
       __builtin_amdgcn_global_load_lds(xb + min(r + half, N - 1) * p.x_node_stride + (c8 < nch ? c8 : 0),
                                        (__attribute__((address_space(3))) void*)(rows + (4 + r) * kConvSlice), 16, 0, 0);
   }
-  if (tid < 4 * N) {
-    const int64_t at = (int64_t)b * p.cidx_req_stride + (int64_t)(tid >> 2) * p.cidx_node_stride + (tid & 3);
-    const int64_t col =
-        CIDX64 ? static_cast<const int64_t*>(p.cidx)[at] : (int64_t) static_cast<const int32_t*>(p.cidx)[at];
-    taps[tid] = col >= 0 && col < 3 + N ? 2 * kConvSlice * (1 + (int)col) : 0;
-  }
+  // one tap column per thread (the low and the high word of a 64-bit one)
+  const int tap = min(tid, 4 * N - 1);
+  const int64_t tap_at = (int64_t)b * p.cidx_req_stride + (int64_t)(tap >> 2) * p.cidx_node_stride + (tap & 3);
+  const int32_t* ci = static_cast<const int32_t*>(p.cidx) + (CIDX64 ? 2 * tap_at : tap_at);
+  const int32_t col_lo = ci[0], col_hi = CIDX64 ? ci[1] : 0;
   const int c0 = 4 * lane;
   const bool active = c0 < nch;
-  float w[16];  // w[4 e + j]: channel c0 + e, tap j
-  {
-    const u32x4* wp = reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(p.weight) +
-                                                     (int64_t)(cbase + (active ? c0 : 0)) * 4);
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const u32x4 u = wp[q];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        w[8 * q + 2 * e] = __uint_as_float(u[e] << 16);
-        w[8 * q + 2 * e + 1] = __uint_as_float(u[e] & 0xffff0000u);
-      }
-    }
+  const u32x4* wp = reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(p.weight) +
+                                                   (int64_t)(cbase + (active ? c0 : 0)) * 4);
+  const u32x4 wraw[2] = {wp[0], wp[1]};
+  // one channel of the state per thread
+  const int chan = min(tid, nch - 1);
+  const uint16_t* cs = static_cast<const uint16_t*>(p.conv_state) + (slot_raw < 0 ? 0 : slot_raw) * p.cs_slot_stride +
+                       (int64_t)(cbase + chan) * p.cs_chan_stride;
+  const uint16_t state[3] = {cs[0], cs[p.cs_col_stride], cs[2 * p.cs_col_stride]};
+  __builtin_amdgcn_sched_barrier(0);
+
+  if (tid < 4 * N) {
+    const int64_t col = CIDX64 ? (int64_t)(((uint64_t)(uint32_t)col_hi << 32) | (uint32_t)col_lo) : (int64_t)col_lo;
+    taps[tid] = col >= 0 && col < 3 + N ? 2 * kConvSlice * (1 + (int)col) : 0;
   }
-  float bias[4];
+  float w[16];  // w[4 e + j]: channel c0 + e, tap j
 #pragma unroll
-  for (int e = 0; e < 4; ++e) bias[e] = p.bias && active ? ld_f(p.bias, cbase + c0 + e, p.bias_dtype) : 0.f;
+  for (int q = 0; q < 2; ++q)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      w[8 * q + 2 * e] = __uint_as_float(wraw[q][e] << 16);
+      w[8 * q + 2 * e + 1] = __uint_as_float(wraw[q][e] & 0xffff0000u);
+    }
   if (tid < nch) {
-    const int64_t slot = slot_raw < 0 ? 0 : slot_raw;
-    const uint16_t* cs = static_cast<const uint16_t*>(p.conv_state) + slot * p.cs_slot_stride +
-                         (int64_t)(cbase + tid) * p.cs_chan_stride;
-    uint16_t h[3];
 #pragma unroll
-    for (int j = 0; j < 3; ++j) h[j] = cs[j * p.cs_col_stride];
+    for (int j = 0; j < 3; ++j) rows[(1 + j) * kConvSlice + tid] = state[j];
+  }
+  float bias[4] = {0.f, 0.f, 0.f, 0.f};
+  if (p.bias) {  // uniform
 #pragma unroll
-    for (int j = 0; j < 3; ++j) rows[(1 + j) * kConvSlice + tid] = h[j];
+    for (int e = 0; e < 4; ++e) bias[e] = active ? ld_f(p.bias, cbase + c0 + e, p.bias_dtype) : 0.f;
   }
   if (tid < 64) *reinterpret_cast<uint2*>(rows + 4 * tid) = uint2{0u, 0u};
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the row copies
