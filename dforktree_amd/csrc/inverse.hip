@@ -15,16 +15,18 @@
 // Bound by memory: 2 n^2 floats per matrix.  2048 64 x 64 matrices (67 MB),
 // with the copy that keeps the input (about 8 us): 44.5 us with one column
 // per lane (each lane read its own 256-byte row, element by element, and ran
-// 2016 dependent multiply-adds), 23.8 us here.  16 KiB of LDS at 64 nodes
-// holds 10 waves per CU, so 2048 matrices are resident at once.
+// 2016 dependent multiply-adds), 23.0 us here.  16 KiB of LDS at 64 nodes
+// holds 10 waves per CU, so 2048 matrices are resident at once, and would
+// load, compute and store in step: so every load goes out first, a block row
+// is solved as soon as its own rows are in and leaves while the next one is
+// solved (4% against copies straight into LDS, waited for at once).
 #include "dft_device.h"
 
 namespace dft {
 namespace {
 
 // 16-byte chunk c / 4 of row i at chunk position (c / 4) ^ i (mod the row's
-// chunks): rows stay contiguous, so one 1 KiB global->LDS load fills whole
-// rows, and the 16-byte reads of 16 rows at one column hit distinct banks
+// chunks): rows stay contiguous, so a wave's 1 KiB is whole rows, and the 16-byte reads of 16 rows at one column hit distinct banks
 // (at 64; 2- and 4-way conflicts at 32 and 16, where there are few reads).
 template <int NP>
 __device__ __forceinline__ int mat_at(int i, int c) {
@@ -62,9 +64,12 @@ __device__ __forceinline__ void subst_steps(const float (&na)[16], f32x4 (&x)[J]
 
 // block row I; xr[m][j]: X_mj of the block rows above as MFMA operands
 // (element s of lane (n, g): X[16m + 4g + s][16j + n])
-template <int NP, int I>
-__device__ __forceinline__ void block_rows(float* a, int n16, int g4, f32x4 (&xr)[NP / 16][NP / 16]) {
+// before(I) runs ahead of block row I, after(I) behind it.
+template <int NP, int I, class Before, class After>
+__device__ __forceinline__ void block_rows(float* a, int n16, int g4, f32x4 (&xr)[NP / 16][NP / 16], Before before,
+                                           After after) {
   if constexpr (I < NP / 16) {
+    before(I);
     f32x4 x[I + 1];
     if constexpr (I > 0) {
       f32x4 am[I];  // A[16I + n][16m + 4g ..]
@@ -102,44 +107,51 @@ __device__ __forceinline__ void block_rows(float* a, int n16, int g4, f32x4 (&xr
 #pragma unroll
         for (int s = 0; s < 4; ++s) xr[I][j][s] = a[mat_at<NP>(16 * I + 4 * g4 + s, 16 * j + n16)];
     }
-    block_rows<NP, I + 1>(a, n16, g4, xr);
+    after(I);
+    block_rows<NP, I + 1>(a, n16, g4, xr, before, after);
   }
 }
 
-// VEC: n == NP and every matrix 16-byte aligned (whole 16-byte pieces, the
-// loads straight into LDS); else row by row, a column per lane.
+// VEC: n == NP and every matrix 16-byte aligned (whole 16-byte pieces); else
+// row by row, a column per lane.
 template <int NP, bool VEC>
 __global__ void __launch_bounds__(64) block_inverse_kernel(float* x, int n, int64_t mat_stride) {
   __shared__ alignas(16) float a[NP * NP];
   constexpr int CH = NP / 4;  // 16-byte chunks of a row
   float* m = x + (int64_t)blockIdx.x * mat_stride;
   const int lane = threadIdx.x;
+  f32x4 xr[NP / 16][NP / 16];
   if constexpr (VEC) {
+    constexpr int PB = NP / 16;  // 1 KiB pieces of whole rows per block row
+    f32x4 ld[PB * PB];
 #pragma unroll
-    for (int b = 0; b < NP * NP / 256; ++b) {  // 1 KiB: rows (64 / CH) b ..
+    for (int b = 0; b < PB * PB; ++b) {
       const int i = (64 / CH) * b + lane / CH;
-      __builtin_amdgcn_global_load_lds(m + i * NP + 4 * ((lane ^ i) & (CH - 1)),
-                                       (__attribute__((address_space(3))) void*)(a + 256 * b), 16, 0, 0);
+      ld[b] = *reinterpret_cast<const f32x4*>(m + i * NP + 4 * ((lane ^ i) & (CH - 1)));
     }
+    block_rows<NP, 0>(
+        a, lane & 15, lane >> 4, xr,
+        [&](int bi) {
+#pragma unroll
+          for (int b = 0; b < PB; ++b) *reinterpret_cast<f32x4*>(&a[256 * (PB * bi + b) + 4 * lane]) = ld[PB * bi + b];
+          asm volatile("" ::: "memory");
+        },
+        [&](int bi) {  // (tiles above the diagonal still hold A: zeros)
+#pragma unroll
+          for (int b = 0; b < PB; ++b) {
+            const int i = (64 / CH) * (PB * bi + b) + lane / CH, c = (lane ^ i) & (CH - 1);
+            const f32x4 v = *reinterpret_cast<const f32x4*>(&a[256 * (PB * bi + b) + 4 * lane]);
+            *reinterpret_cast<f32x4*>(m + i * NP + 4 * c) = (c >> 2) > (i >> 4) ? f32x4{} : v;
+          }
+        });
   } else {
 #pragma unroll 16
     for (int i = 0; i < NP; ++i) {
       const float v = (i < n && lane < n) ? m[i * n + lane] : 0.f;
       if (lane < NP) a[mat_at<NP>(i, lane)] = v;
     }
-  }
-  __syncthreads();
-  f32x4 xr[NP / 16][NP / 16];
-  block_rows<NP, 0>(a, lane & 15, lane >> 4, xr);
-  // tiles above the diagonal still hold A: zeros
-  if constexpr (VEC) {
-#pragma unroll
-    for (int b = 0; b < NP * NP / 256; ++b) {
-      const int i = (64 / CH) * b + lane / CH, c = (lane ^ i) & (CH - 1);
-      const f32x4 v = *reinterpret_cast<const f32x4*>(&a[256 * b + 4 * lane]);
-      *reinterpret_cast<f32x4*>(m + i * NP + 4 * c) = (c >> 2) > (i >> 4) ? f32x4{} : v;
-    }
-  } else {
+    __syncthreads();
+    block_rows<NP, 0>(a, lane & 15, lane >> 4, xr, [](int) {}, [](int) {});
     if (lane < n)
       for (int i = 0; i < n; ++i) m[i * n + lane] = (lane >> 4) > (i >> 4) ? 0.f : a[mat_at<NP>(i, lane)];
   }
