@@ -2771,18 +2771,19 @@ static bool mixed_launch(const dft_verify_args* a, bool split) {
 // item's value columns over two workgroups: each forms phase 1 in full and
 // phases 2-3, the state read and the stores on half the columns, which
 // shortens a workgroup's life where the launch is latency-bound.
+//  * the plain verify + commit, 12 layers: 9 requests (288 items) 227 -> 221
+//    us, 12 (384) 259 -> 256, 14 (448) 277 -> 296;
+//  * the fused commit -> verify, 24 layers: batch 1 (32 items) 367 -> 297 us,
+//    batch 4 (27 nodes) 414 -> 341, batch 8 432 -> 407, batch 12 (384) 530 ->
+//    512, batch 16 (512) 545 -> 763: three of its workgroups fit a CU, by LDS
+//    and registers, 768 in one generation.  The split halves hold half the
+//    tile's registers, which also makes room for the whole-wave diagonal
+//    solves (367 -> 348 us at batch 4), and take their v rows with the q/k
+//    rows instead of behind the write-back.
 // Launches over 32 nodes with at most kSplitItems64 items do the same with
 // the 64-wide kernel (tail_halves; 110 KiB of LDS, one workgroup per CU, so
 // at most 256 workgroups for the 256 CUs).
-// The fused commit -> verify of up to 32 nodes splits its columns the same
-// way up to kSplitItemsFused items (three of its workgroups fit a CU, by LDS
-// and registers: 768 in one generation).  24 layers: batch 1 (32 items) 367
-// -> 297 us, batch 4 (27 nodes) 414 -> 341, batch 8 432 -> 407, batch 12 530
-// -> 512; batch 16 (512 items) would go from 545 to 763.  The split halves
-// hold half the tile's registers, which also makes room for the whole-wave
-// diagonal solves (367 -> 348 us at batch 4), and take their v rows with the
-// q/k rows instead of behind the write-back.
-constexpr int kSplitItems = 256, kSplitItems64 = 128, kSplitItemsFused = 384;
+constexpr int kSplitItems = 384, kSplitItems64 = 128;
 
 int launch_tree_verify(const dft_verify_args* a, hipStream_t stream) {
   const VerifyParams P = make_params(a);
@@ -2861,11 +2862,11 @@ int launch_tree_commit_verify(const dft_verify_args* a, const dft_pending_commit
   }
   if (a->n_nodes > 32) DFT_FUSED(64, 1, grid, block64, wide)
   if (a->n_nodes <= 32 || split) {
-    if (pdma && items <= kSplitItemsFused)
+    if (pdma && items <= kSplitItems)
       hipLaunchKernelGGL((tree_commit_verify_kernel<32, true, true, true, 2>), grid2, block, 0, stream, narrow);
     else if (pdma)
       hipLaunchKernelGGL((tree_commit_verify_kernel<32, true, true, true>), grid, block, 0, stream, narrow);
-    else if (items <= kSplitItemsFused)
+    else if (items <= kSplitItems)
       DFT_FUSED(32, 2, grid2, block, narrow)
     else
       DFT_FUSED(32, 1, grid, block, narrow)
