@@ -142,36 +142,40 @@ __global__ void __launch_bounds__(256) tree_struct_kernel(const dft_tree_args p,
 }
 
 // Dense 0/1 ancestry rows -> the uint64 rows the verify and commit read.
-// One wave per request: lane j loads column j of every row first (coalesced
-// rows, all loads in flight at once), then the wave's ballot of each row is
-// that row's mask; bits above the diagonal are dropped, as the kernels that
-// read dense rows drop them.  Lane i keeps row i and writes it at the end.
+// Four waves per request, each with 16 of the rows (one wave with all 64: 2 to
+// 3 us more per batch-1 step): lane j loads column j of
+// every one of them first (coalesced rows, all loads in flight at once), then
+// the wave's ballot of each row is that row's mask; bits above the diagonal
+// are dropped, as the kernels that read dense rows drop them.  Lane i keeps
+// the wave's row i and writes it at the end.
 // The loads take clamped, always valid addresses (row and column min(., n-1))
 // and the ballots mask what lies outside the n x n matrix: with the bounds in
 // a condition around each load, every load sat in its own branch and was
 // waited for at once (batch 1: 7.4 us per launch at 32 nodes).
-__global__ void __launch_bounds__(256) anc_pack_kernel(const dft_anc_pack_args p) {
-  const int lane = threadIdx.x & 63;
-  const int b = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (b >= p.batch) return;  // no barrier in this kernel
+__device__ __forceinline__ void anc_pack_request(const dft_anc_pack_args& p, int b) {
+  const int lane = threadIdx.x & 63, r0 = 16 * (threadIdx.x >> 6);
   const int n = p.n_nodes;
-  if (n <= 0) return;        // (uniform) no rows
+  if (r0 >= n) return;  // (uniform over the wave) no rows
   const float* base = p.anc + (int64_t)b * p.anc_req_stride + (lane < n ? lane : n - 1);
-  float v[64];
+  float v[16];
 #pragma unroll
-  for (int i = 0; i < 64; ++i) v[i] = base[(int64_t)(i < n ? i : n - 1) * p.anc_row_stride];
+  for (int i = 0; i < 16; ++i) v[i] = base[(int64_t)(r0 + i < n ? r0 + i : n - 1) * p.anc_row_stride];
   const bool col_in = lane < n;
   uint64_t mine = 0;
 #pragma unroll
-  for (int i = 0; i < 64; ++i) {
-    const uint64_t row = i < n ? __ballot(col_in && v[i] > 0.5f) & mask_upto(i) : 0ull;
+  for (int i = 0; i < 16; ++i) {
+    const uint64_t row = __ballot(col_in && v[i] > 0.5f) & mask_upto(r0 + i);
     if (lane == i) mine = row;
   }
-  if (lane < n) p.anc_bits[(int64_t)b * n + lane] = mine;
+  if (lane < 16 && r0 + lane < n) p.anc_bits[(int64_t)b * n + r0 + lane] = mine;
+}
+
+__global__ void __launch_bounds__(256) anc_pack_kernel(const dft_anc_pack_args p) {
+  for (int b = blockIdx.x; b < p.batch; b += gridDim.x) anc_pack_request(p, b);
 }
 
 int launch_anc_pack(const dft_anc_pack_args* a, hipStream_t stream) {
-  const dim3 grid((unsigned)((a->batch + 3) / 4));
+  const dim3 grid((unsigned)(a->batch < 65536 ? a->batch : 65536));  // workgroups stride over further requests
   hipLaunchKernelGGL(anc_pack_kernel, grid, dim3(256), 0, stream, *a);
   return hipGetLastError() == hipSuccess ? DFT_OK : DFT_ERR_LAUNCH;
 }
