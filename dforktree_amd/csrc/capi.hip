@@ -192,7 +192,7 @@ int dft_anc_pack(const dft_anc_pack_args* a, void* stream) {
   if (!a) return DFT_ERR_INVALID;
   if (a->batch < 0 || a->n_nodes < 0 || a->n_nodes > 64) return DFT_ERR_INVALID;
   if (a->batch == 0 || a->n_nodes == 0) return DFT_OK;
-  if (((int64_t)a->batch + 3) / 4 > max_blocks(256)) return DFT_ERR_UNSUPPORTED;  // a wave per request
+  if (((int64_t)a->batch + 3) / 4 > max_blocks(256)) return DFT_ERR_UNSUPPORTED;
   if (!a->anc || !a->anc_bits) return DFT_ERR_INVALID;
   return dft::launch_anc_pack(a, static_cast<hipStream_t>(stream));
 }

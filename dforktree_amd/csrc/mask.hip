@@ -10,8 +10,7 @@
 // request's mask) starts at the byte offset sum_{s' < s} ceil(bits_s' / 8);
 // every workgroup of a segment computes that sum itself (a block reduction
 // over the earlier segments' sizes), so one launch suffices and nothing is
-// read back by the host.  A thread produces an aligned word (packbits) or
-// 16-byte piece (mask) of the output.
+// read back by the host.  A thread produces an aligned word of the output.
 #include <stdint.h>
 
 #include "dft_device.h"
@@ -183,14 +182,18 @@ __device__ __forceinline__ uint32_t row_bits(uint64_t anc, int64_t plen, int64_t
   return low_mask(k) | ((uint32_t)(anc << k) & low_mask(take));
 }
 
-// A thread produces one aligned 16-byte piece of the output (a piece that
-// the segment's ends or the capacity cut is stored word by word and byte by
-// byte).  Most pieces lie inside one row's prefix: all ones.  The ancestry
-// rows are read once per workgroup.  With one 32-bit word of the segment's
-// own stream per thread (a division each, the ancestry row read per word,
-// and byte stores wherever a segment starts at an odd byte) the launch took
-// 8.7 us for 64 requests of 16-64 nodes and about 6000 tokens (2 MB), now
-// 6.6 us, most of it the dependent loads in front of the first store.
+// A thread produces one aligned word of the output (a word that the
+// segment's ends or the capacity cut is stored byte by byte).  Most words lie
+// inside one row's prefix: all ones.  The ancestry rows are read once per
+// workgroup, and there is a thread per word of the capacity, where 8
+// workgroups per segment walked its words with a division and an ancestry
+// read each, and stored bytes wherever a segment starts at an odd one.  us
+// per launch, back to back, before and now (2 words a thread, 4 words):
+//   64 requests x 32 nodes, 4096 tokens          4.0   4.1 (4.5, 5.6)
+//   64 x 16-64 nodes, about 6000 tokens          7.8   5.6 (5.2, 6.0)
+//   1 x 64 nodes, 32768 tokens                  12.3   2.8 (3.0, 3.4)
+//   8 x 8-64 nodes, about 20000 tokens          12.5   3.6 (4.2, 5.2)
+//   128 x 8-64 nodes, about 300 tokens           3.9   4.0 (5.0, 4.9)
 __global__ void __launch_bounds__(kThreads) tree_mask_kernel(const dft_mask_args a) {
   __shared__ int64_t red[kThreads / 64];
   __shared__ uint64_t anc[64];
@@ -205,12 +208,12 @@ __global__ void __launch_bounds__(kThreads) tree_mask_kernel(const dft_mask_args
     store_indptr(a.out_indptr, a.out_indptr_dtype, b, off);
     if (b + 1 == (int)gridDim.y) store_indptr(a.out_indptr, a.out_indptr_dtype, b + 1, off + nbytes);
   }
-  const int lead = (int)(reinterpret_cast<uintptr_t>(a.out + off) & 15);  // bytes of piece 0 in front of the segment
-  const int64_t pieces = nbytes > 0 ? (lead + nbytes + 15) >> 4 : 0;
+  const int lead = (int)(reinterpret_cast<uintptr_t>(a.out + off) & 3);  // bytes of word 0 in front of the segment
+  const int64_t nwords = nbytes > 0 ? (lead + nbytes + 3) >> 2 : 0;
   bool ok = true;
-  for (int64_t w = (int64_t)blockIdx.x * kThreads + threadIdx.x; w < pieces; w += (int64_t)gridDim.x * kThreads) {
-    const int64_t j = 16 * w - lead;         // byte of the segment
-    int skip = j < 0 ? (int)(-8 * j) : 0;    // bits of the piece in front of the segment
+  for (int64_t w = (int64_t)blockIdx.x * kThreads + threadIdx.x; w < nwords; w += (int64_t)gridDim.x * kThreads) {
+    const int64_t j = 4 * w - lead;       // byte of the segment
+    int done = j < 0 ? (int)(-8 * j) : 0;  // bits of the word in front of the segment
     const int64_t q0 = j < 0 ? 0 : 8 * j;
     int64_t r, c;
     if (nbits <= 0x7fffffff) {  // 32-bit division (uniform per request)
@@ -220,34 +223,20 @@ __global__ void __launch_bounds__(kThreads) tree_mask_kernel(const dft_mask_args
       r = q0 / L;
       c = q0 - r * L;
     }
-    u32x4 piece;
-    if (skip == 0 && c + 128 <= m.plen) {
-      piece = u32x4{~0u, ~0u, ~0u, ~0u};
+    uint32_t word = 0;
+    if (done == 0 && c + 32 <= m.plen) {
+      word = ~0u;
     } else {
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        uint32_t word = 0;
-        int done = skip > 32 ? 32 : skip;
-        skip -= done;
-        while (done < 32 && r < m.n) {  // at most 32 rows (rows are >= 1 bit long)
-          const int take = (int)(L - c < 32 - done ? L - c : 32 - done);
-          word |= row_bits(anc[r], m.plen, c, take) << done;
-          done += take;
-          c += take;
-          if (c == L) {
-            ++r;
-            c = 0;
-          }
-        }
-        piece[k] = to_order(word, a.bit_order);
+      while (done < 32 && r < m.n) {  // at most 32 rows (rows are >= 1 bit long)
+        const int take = (int)(L - c < 32 - done ? L - c : 32 - done);
+        word |= row_bits(anc[r], m.plen, c, take) << done;
+        done += take;
+        ++r;
+        c = 0;
       }
+      word = to_order(word, a.bit_order);
     }
-    if (j >= 0 && j + 16 <= nbytes && off + j + 16 <= a.out_capacity) {
-      *reinterpret_cast<u32x4*>(a.out + off + j) = piece;
-    } else {
-#pragma unroll
-      for (int k = 0; k < 4; ++k) ok &= store_word(a.out, a.out_capacity, off, nbytes, j + 4 * k, piece[k]);
-    }
+    ok &= store_word(a.out, a.out_capacity, off, nbytes, j, word);
   }
   if (!ok && a.status) *a.status = 1;
 }
@@ -267,11 +256,11 @@ int launch_packbits(const dft_packbits_args* a, hipStream_t stream) {
 }
 
 int launch_tree_mask(const dft_mask_args* a, hipStream_t stream) {
-  // the sizes stay on the device: one thread per 16-byte piece if the
-  // requests share the output's capacity evenly (they stride otherwise), up
-  // to a chip's worth of workgroups
+  // the sizes stay on the device: one thread per word if the requests share
+  // the output's capacity evenly (they stride otherwise), up to a chip's worth
+  // of workgroups
   const int64_t most = a->batch < 2048 ? 2048 / a->batch : 1;
-  const int64_t need = (a->out_capacity / a->batch + 16 * kThreads - 1) / (16 * kThreads);
+  const int64_t need = (a->out_capacity / a->batch + 4 * kThreads - 1) / (4 * kThreads);
   const int64_t bx = need < 1 ? 1 : (need > most ? most : need);
   hipLaunchKernelGGL(tree_mask_kernel, dim3((unsigned)bx, (unsigned)a->batch), dim3(kThreads), 0, stream, *a);
   return hipGetLastError() == hipSuccess ? DFT_OK : DFT_ERR_LAUNCH;

@@ -139,7 +139,7 @@ def test_plan_override_packs_on_the_device(cuda, monkeypatch):
 
 
 # the elements start 0-5 bytes past an aligned address (whole dwords, shifted
-# dwords), the bytes 0-17 past one (cut words and 16-byte pieces at both ends)
+# dwords), the bytes 0-17 past one (cut words at both ends)
 @pytest.mark.parametrize("x_off,out_off", [(0, 0), (1, 0), (2, 3), (3, 16), (4, 1), (5, 7)])
 @pytest.mark.parametrize("bitorder", ["little", "big"])
 def test_packbits_alignment(cuda, x_off, out_off, bitorder):
@@ -162,7 +162,7 @@ def test_packbits_alignment(cuda, x_off, out_off, bitorder):
 @pytest.mark.parametrize("out_off", [0, 1, 4, 15])
 @pytest.mark.parametrize("bitorder", ["little", "big"])
 def test_tree_mask_alignment(cuda, out_off, bitorder):
-    """Segments at every byte alignment, rows shorter and longer than a 16-byte piece, one workgroup and many."""
+    """Segments at every byte alignment, rows shorter and longer than a word, one workgroup and many."""
     from dforktree_amd import ops
     sizes = [1, 2, 3, 31, 64, 33, 5, 64, 16]
     kinds = ["chain", "bushy", "random"] * 3
