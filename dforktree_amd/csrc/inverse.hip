@@ -10,7 +10,11 @@
 // 16-lane row (one DPP row broadcast, fused into the multiply-add) and each
 // lane's own A[16i + n][16i + m], so the tiles of a block row share one
 // register per step and run side by side.  The sums are the forward
-// substitution's own, with no product by an inverted diagonal block.
+// substitution's own, with no product by an inverted diagonal block, and a
+// non-finite value goes where it goes there: into its own row of X and the
+// rows below that use it, never into the rows above (subst_step).  An element
+// A[i][c] that is itself not finite takes in every column of row i up to the
+// end of c's 16-column block, as 0 * NaN.
 //
 // Bound by memory: 2 n^2 floats per matrix.  2048 64 x 64 matrices (67 MB),
 // with the copy that keeps the input (about 8 us): 44.5 us with one column
@@ -33,31 +37,55 @@ __device__ __forceinline__ int mat_at(int i, int c) {
   return i * NP + ((((c >> 2) ^ i) & (NP / 4 - 1)) << 2) + (c & 3);
 }
 
-// Step M of the substitution on one tile: x[r] += na * (x[r] of lane M of the
-// 16-lane row).  The compiler keeps the broadcast as a move of its own (with
-// two wait states after each multiply-add), hence the statement; the two
-// wait states a DPP read needs after a vector write lie in the s_nop for the
-// first instruction and in the three others for the rest.  x must not come
-// straight from an MFMA: the backend does not see the reads in here.
-template <int M>
-__device__ __forceinline__ void subst_step(float na, f32x4& x) {
-  float x0 = x[0], x1 = x[1], x2 = x[2], x3 = x[3];
-  asm("s_nop 1\n\t"
-      "v_fmac_f32_dpp %0, %0, %4 row_newbcast:%c5 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %1, %1, %4 row_newbcast:%c5 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %2, %2, %4 row_newbcast:%c5 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %3, %3, %4 row_newbcast:%c5 row_mask:0xf bank_mask:0xf"
-      : "+v"(x0), "+v"(x1), "+v"(x2), "+v"(x3)
-      : "v"(na), "i"(M));
-  x = f32x4{x0, x1, x2, x3};
+// Step M of the substitution on the J tiles of a block row: x += na * (x of
+// lane M of the 16-lane row), on the lanes from M on.  The lanes below M are
+// masked off and lane M's own na is the smallest normal number (x + 2^-126 x
+// is x, also for infinities), where zeros would do for finite values: 0 * inf
+// and 0 * NaN would carry a bad row M back into the finished rows above it.
+// The compiler keeps the broadcast as a move of its own (with two wait states
+// after each multiply-add), hence the statement; the two wait states a DPP
+// read needs after a vector write are the two moves to the lane mask for the
+// first instruction and lie in the three others for the rest.  Every lane of
+// the wave is active here.  x must not come straight from an MFMA: the backend
+// does not see the reads in here.
+#define DFT_STEP4(a, b, c, d) DFT_STEP1(a) DFT_STEP1(b) DFT_STEP1(c) DFT_STEP1(d)
+#define DFT_STEP1(k) "v_fmac_f32_dpp %" #k ", %" #k ", %[na] row_newbcast:%c[m] row_mask:0xf bank_mask:0xf\n\t"
+#define DFT_STEP_OUT(j) "+v"(t[j][0]), "+v"(t[j][1]), "+v"(t[j][2]), "+v"(t[j][3])
+#define DFT_STEP(text, ...)                                                                      \
+  asm("s_mov_b32 exec_lo, %[lanes]\n\ts_mov_b32 exec_hi, %[lanes]\n\t" text "s_mov_b64 exec, -1" \
+      : __VA_ARGS__                                                                              \
+      : [na] "v"(na), [m] "i"(M), [lanes] "i"((int32_t)kLanes))
+template <int M, int J>
+__device__ __forceinline__ void subst_step(float na, f32x4 (&x)[J]) {
+  constexpr uint32_t kLanes = ((0xffffu << M) & 0xffffu) * 0x00010001u;  // of each half wave
+  float t[J][4];
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) t[j][r] = x[j][r];
+  if constexpr (J == 1)
+    DFT_STEP(DFT_STEP4(0, 1, 2, 3), DFT_STEP_OUT(0));
+  else if constexpr (J == 2)
+    DFT_STEP(DFT_STEP4(0, 1, 2, 3) DFT_STEP4(4, 5, 6, 7), DFT_STEP_OUT(0), DFT_STEP_OUT(1));
+  else if constexpr (J == 3)
+    DFT_STEP(DFT_STEP4(0, 1, 2, 3) DFT_STEP4(4, 5, 6, 7) DFT_STEP4(8, 9, 10, 11), DFT_STEP_OUT(0), DFT_STEP_OUT(1),
+             DFT_STEP_OUT(2));
+  else
+    DFT_STEP(DFT_STEP4(0, 1, 2, 3) DFT_STEP4(4, 5, 6, 7) DFT_STEP4(8, 9, 10, 11) DFT_STEP4(12, 13, 14, 15),
+             DFT_STEP_OUT(0), DFT_STEP_OUT(1), DFT_STEP_OUT(2), DFT_STEP_OUT(3));
+#pragma unroll
+  for (int j = 0; j < J; ++j) x[j] = f32x4{t[j][0], t[j][1], t[j][2], t[j][3]};
 }
+#undef DFT_STEP
+#undef DFT_STEP_OUT
+#undef DFT_STEP1
+#undef DFT_STEP4
 
 // steps M .. 14 on tiles 0 .. J - 1 of a block row
 template <int M, int J>
 __device__ __forceinline__ void subst_steps(const float (&na)[16], f32x4 (&x)[J]) {
   if constexpr (M < 15) {
-#pragma unroll
-    for (int j = 0; j < J; ++j) subst_step<M>(na[M], x[j]);
+    subst_step<M>(na[M], x);
     subst_steps<M + 1, J>(na, x);
   }
 }
@@ -87,12 +115,12 @@ __device__ __forceinline__ void block_rows(float* a, int n16, int g4, f32x4 (&xr
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) x[I][r] = (n16 == 4 * g4 + r) ? 1.f : 0.f;
-    float na[16];  // the strict lower part of row n of A_II, negated
+    float na[16];  // row n of A_II, negated, and subst_step's diagonal (what lies above that meets no active lane)
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       const f32x4 v = *reinterpret_cast<const f32x4*>(&a[mat_at<NP>(16 * I + n16, 16 * I + 4 * c)]);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) na[4 * c + e] = 4 * c + e < n16 ? -v[e] : 0.f;
+      for (int e = 0; e < 4; ++e) na[4 * c + e] = 4 * c + e == n16 ? 0x1p-126f : -v[e];
     }
     subst_steps<0, I + 1>(na, x);
     // over A's rows 16I .., which nothing reads any more (one wave: its LDS
