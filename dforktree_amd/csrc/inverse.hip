@@ -30,8 +30,9 @@ namespace dft {
 namespace {
 
 // 16-byte chunk c / 4 of row i at chunk position (c / 4) ^ i (mod the row's
-// chunks): rows stay contiguous, so a wave's 1 KiB is whole rows, and the 16-byte reads of 16 rows at one column hit distinct banks
-// (at 64; 2- and 4-way conflicts at 32 and 16, where there are few reads).
+// chunks): rows stay contiguous, so a wave's 1 KiB is whole rows, and the
+// 16-byte reads of 16 rows at one column hit distinct banks (at 64; 2- and
+// 4-way conflicts at 32 and 16, where there are few reads).
 template <int NP>
 __device__ __forceinline__ int mat_at(int i, int c) {
   return i * NP + ((((c >> 2) ^ i) & (NP / 4 - 1)) << 2) + (c & 3);
@@ -140,22 +141,28 @@ __device__ __forceinline__ void block_rows(float* a, int n16, int g4, f32x4 (&xr
   }
 }
 
-// VEC: n == NP and every matrix 16-byte aligned (whole 16-byte pieces); else
-// row by row, a column per lane.
-template <int NP, bool VEC>
+// 16 bytes of a matrix: its floats are aligned, its rows need not be
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
+// WHOLE: n == NP, the matrix moves as 16-byte pieces; else as 64 / NP rows of
+// NP floats per load, the elements past n left out.  us for 2048 matrices in
+// cache, a row per load and store in turn (which an unaligned whole matrix
+// took too) and now: 20 x 20 8.3 / 5.0, 33 x 33 16.1 / 12.9, 48 x 48 18.7 /
+// 14.0; unaligned 16 x 16 6.2 / 3.4, 32 x 32 10.6 / 4.7, 64 x 64 23.6 / 10.9.
+template <int NP, bool WHOLE>
 __global__ void __launch_bounds__(64) block_inverse_kernel(float* x, int n, int64_t mat_stride) {
   __shared__ alignas(16) float a[NP * NP];
   constexpr int CH = NP / 4;  // 16-byte chunks of a row
   float* m = x + (int64_t)blockIdx.x * mat_stride;
   const int lane = threadIdx.x;
   f32x4 xr[NP / 16][NP / 16];
-  if constexpr (VEC) {
+  if constexpr (WHOLE) {
     constexpr int PB = NP / 16;  // 1 KiB pieces of whole rows per block row
     f32x4 ld[PB * PB];
 #pragma unroll
     for (int b = 0; b < PB * PB; ++b) {
       const int i = (64 / CH) * b + lane / CH;
-      ld[b] = *reinterpret_cast<const f32x4*>(m + i * NP + 4 * ((lane ^ i) & (CH - 1)));
+      ld[b] = *reinterpret_cast<const f32x4_a4*>(m + i * NP + 4 * ((lane ^ i) & (CH - 1)));
     }
     block_rows<NP, 0>(
         a, lane & 15, lane >> 4, xr,
@@ -169,26 +176,38 @@ __global__ void __launch_bounds__(64) block_inverse_kernel(float* x, int n, int6
           for (int b = 0; b < PB; ++b) {
             const int i = (64 / CH) * (PB * bi + b) + lane / CH, c = (lane ^ i) & (CH - 1);
             const f32x4 v = *reinterpret_cast<const f32x4*>(&a[256 * (PB * bi + b) + 4 * lane]);
-            *reinterpret_cast<f32x4*>(m + i * NP + 4 * c) = (c >> 2) > (i >> 4) ? f32x4{} : v;
+            *reinterpret_cast<f32x4_a4*>(m + i * NP + 4 * c) = (c >> 2) > (i >> 4) ? f32x4{} : v;
           }
         });
   } else {
-#pragma unroll 16
-    for (int i = 0; i < NP; ++i) {
-      const float v = (i < n && lane < n) ? m[i * n + lane] : 0.f;
-      if (lane < NP) a[mat_at<NP>(i, lane)] = v;
-    }
-    __syncthreads();
+    // (the loads take clamped, always valid addresses and go out together)
+    constexpr int RL = 64 / NP, K = NP / RL, G = K < 16 ? K : 16;  // rows per load, loads, loads per group
+    const int r0 = lane / NP, c = lane & (NP - 1);
+    float v[K] = {};
+#pragma unroll
+    for (int k = 0; k < K; k += G)
+      if (RL * k < n)  // uniform
+#pragma unroll
+        for (int e = k; e < k + G; ++e) v[e] = m[min(RL * e + r0, n - 1) * n + min(c, n - 1)];
+#pragma unroll
+    for (int k = 0; k < K; ++k) a[mat_at<NP>(RL * k + r0, c)] = max(RL * k + r0, c) < n ? v[k] : 0.f;
+    asm volatile("" ::: "memory");
     block_rows<NP, 0>(a, lane & 15, lane >> 4, xr, [](int) {}, [](int) {});
-    if (lane < n)
-      for (int i = 0; i < n; ++i) m[i * n + lane] = (lane >> 4) > (i >> 4) ? 0.f : a[mat_at<NP>(i, lane)];
+#pragma unroll
+    for (int k = 0; k < K; k += G)
+      if (RL * k < n) {
+#pragma unroll
+        for (int e = k; e < k + G; ++e) v[e] = a[mat_at<NP>(RL * e + r0, c)];
+#pragma unroll
+        for (int e = k; e < k + G; ++e)
+          if (max(RL * e + r0, c) < n) m[(RL * e + r0) * n + c] = (c >> 4) > ((RL * e + r0) >> 4) ? 0.f : v[e];
+      }
   }
 }
 
 template <int NP>
 void launch(float* x, int n_mats, int n, int64_t mat_stride, hipStream_t stream) {
-  const bool vec = n == NP && reinterpret_cast<uintptr_t>(x) % 16 == 0 && mat_stride % 4 == 0;
-  if (vec)
+  if (n == NP)
     hipLaunchKernelGGL((block_inverse_kernel<NP, true>), dim3(n_mats), dim3(64), 0, stream, x, n, mat_stride);
   else
     hipLaunchKernelGGL((block_inverse_kernel<NP, false>), dim3(n_mats), dim3(64), 0, stream, x, n, mat_stride);

@@ -25,7 +25,7 @@ def _matrices(rng, mats, n):
 
 
 # whole tiles (16-byte pieces), sizes on both sides of a tile, one row; offset:
-# floats the buffer starts past a 16-byte boundary (row-by-row form)
+# floats the buffer starts past a 16-byte boundary
 @pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 31, 32, 33, 47, 48, 63, 64])
 @pytest.mark.parametrize("offset", [0, 1])
 def test_block_inverse_sizes(cuda, n, offset):
