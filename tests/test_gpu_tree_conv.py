@@ -112,32 +112,72 @@ def test_tree_struct_any_parents(cuda, kc, dt):
     assert (h["anc_bits"][cu[9] + 64:cu[10]] == 0).all()
 
 
-@pytest.mark.parametrize("n_nodes", [3, 17, 64])
-def test_tree_struct_fills_what_no_tree_covers(cuda, n_nodes):
+# requests: few, more than one load per thread of the search for the batch's
+# ends, and enough for a wave each; sets only: a wave each at any batch
+@pytest.mark.parametrize("n_nodes,batch,dense", [(3, 5, True), (17, 5, True), (64, 5, True), (64, 5, False),
+                                                 (9, 700, True), (9, 700, False), (5, 4101, True), (64, 4099, False)])
+def test_tree_struct_fills_what_no_tree_covers(cuda, n_nodes, batch, dense):
     """Rows in front of, behind and between the requests, and the dense
-    matrices outside the trees, are zeros on memory that held something else;
-    a request past n_nodes stays inside its own matrix."""
-    from dforktree_amd import ops
-    announce(f"tree_struct fill n_nodes={n_nodes}")
-    sizes, lead, tail = [2, 0, n_nodes, 1, n_nodes + 9], 5, 300
+    matrices outside the trees, are zeros on memory that held something else,
+    and nothing past either is written; a request past n_nodes stays inside
+    its own matrix."""
+    import ctypes
+    from dforktree_amd import _lib
+    announce(f"tree_struct fill n_nodes={n_nodes} batch={batch} dense={dense}")
+    g = np.random.default_rng(batch + n_nodes)
+    sizes = [2, 0, n_nodes, 1, n_nodes + 9] + g.integers(0, n_nodes + 10, batch - 5).tolist()
+    lead, tail, guard = 5, 300, 64
     cu = np.cumsum([lead] + sizes)
     rows = int(cu[-1]) + tail
-    parent = torch.zeros(rows, dtype=torch.int32, device=cuda)  # stars
-    parent[cu[:-1].tolist()] = -1
-    for shape, dt in (((rows,), torch.int64), ((len(sizes), n_nodes, n_nodes), torch.float32)):
-        torch.full(shape, -3, dtype=dt, device=cuda)  # what the allocator hands out again
-    r = ops.tree_struct(parent, 4, cu_seqlens=torch.tensor(cu, dtype=torch.int32).to(cuda), n_nodes=n_nodes,
-                        batch=len(sizes), want=("anc_bits", "anc"))
-    bits, anc = r["anc_bits"].cpu().numpy(), r["anc"].cpu().numpy()
-    want = np.zeros(rows, np.uint64)
-    dense = np.zeros((len(sizes), n_nodes, n_nodes), np.float32)
+    parent = torch.zeros(rows + 1, dtype=torch.int32, device=cuda)  # stars
+    parent[torch.from_numpy(cu[:-1]).to(cuda)] = -1
+    cut = torch.from_numpy(cu.astype(np.int32)).to(cuda)
+    bits = torch.full((rows + guard,), -3, dtype=torch.int64, device=cuda)
+    anc = torch.full((batch * n_nodes * n_nodes + guard,), -3.0, device=cuda)
+    a = _lib.TreeArgs()
+    a.batch, a.n_nodes, a.kc = batch, n_nodes, 4
+    a.parent, a.parent_dtype, a.cu_seqlens, a.anc_bits = parent.data_ptr(), _lib.DFT_I32, cut.data_ptr(), bits.data_ptr()
+    if dense:
+        a.anc_f32, a.anc_row_stride, a.anc_req_stride = anc.data_ptr(), n_nodes, n_nodes * n_nodes
+    stream = torch.cuda.current_stream().cuda_stream
+    assert _lib.load().dft_tree_struct_filled(ctypes.byref(a), rows, stream) == _lib.DFT_OK
+    torch.cuda.synchronize()
+    want = np.zeros(rows + guard, np.uint64)
+    want[rows:] = np.uint64(2 ** 64 - 3)
+    full = np.zeros((batch, n_nodes, n_nodes), np.float32)
     for b, n in enumerate(sizes):
-        for i in range(min(n, 64)):
-            want[cu[b] + i] = (1 << i) | 1
-            if i < n_nodes:
-                dense[b, i, 0] = dense[b, i, i] = 1
-    assert np.array_equal(bits.view(np.uint64), want)
-    assert np.array_equal(anc, dense)
+        i = np.arange(min(n, 64))
+        want[cu[b] + i] = (np.uint64(1) << i.astype(np.uint64)) | np.uint64(1)
+        i = i[:n_nodes]
+        full[b, i, 0] = full[b, i, i] = 1
+    assert np.array_equal(bits.cpu().numpy().view(np.uint64), want)
+    got = anc.cpu().numpy()
+    assert np.array_equal(got[:full.size].reshape(full.shape), full if dense else np.full_like(full, -3))
+    assert np.all(got[full.size:] == -3)
+
+
+def test_tree_struct_a_wave_per_request(cuda):
+    """A batch with a wave per request against the same requests in halves,
+    which take four: every output, malformed parents too."""
+    from dforktree_amd import ops
+    announce("tree_struct wave per request")
+    g = np.random.default_rng(11)
+    batch, half = 4098, 2049
+    sizes = g.integers(0, 65, batch)
+    cu = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    rows = int(cu[-1])
+    local = np.concatenate([np.arange(n) for n in sizes])
+    parent = (g.random(rows) * local).astype(np.int32)
+    parent[g.random(rows) < 0.002] = 40  # a cycle, a later parent, or one past the tree
+    parent = torch.from_numpy(parent).to(cuda)
+    whole = ops.tree_struct(parent, 4, cu_seqlens=torch.from_numpy(cu).to(cuda), n_nodes=64, batch=batch)
+    lo = ops.tree_struct(parent[:cu[half]], 4, cu_seqlens=torch.from_numpy(cu[:half + 1]).to(cuda), n_nodes=64, batch=half)
+    hi = ops.tree_struct(parent[cu[half]:], 4, cu_seqlens=torch.from_numpy(cu[half:] - cu[half]).to(cuda), n_nodes=64,
+                         batch=batch - half)
+    torch.cuda.synchronize()
+    assert int(whole["status"].max()) == 2
+    for k in whole:
+        assert torch.equal(whole[k], torch.cat([lo[k], hi[k]])), k
 
 
 def test_builder_tree_struct_matches_reference_closure(cuda):
@@ -304,7 +344,7 @@ def test_conv_negative_slots(cuda, layout):
         assert np.all(got[untouched] == 5.0), f"window slot {untouched} was written"
 
 
-@pytest.mark.parametrize("n", [1, 20, 32, 64])
+@pytest.mark.parametrize("n", [1, 16, 17, 20, 32, 33, 64])
 def test_anc_pack_matches_oracle_bits(cuda, n):
     """dft_anc_pack: the dense ancestry (as tree_struct / the builder give it)
     packed into bit rows, bit-exact against the oracle's rows (bit 63 is the
