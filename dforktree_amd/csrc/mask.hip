@@ -20,6 +20,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kBlocksPerSegment = 8;  // workgroups per packbits segment (grid-stride over its words)
+constexpr int64_t kMaskBlocks = 768, kMaskWide = 1024;  // launch_tree_mask
 
 __device__ __forceinline__ uint32_t low_mask(int bits) { return bits >= 32 ? 0xffffffffu : ((1u << bits) - 1u); }
 
@@ -28,7 +29,8 @@ __device__ __forceinline__ uint32_t to_order(uint32_t w, int order) {
   return order == DFT_BITS_BIG ? __builtin_bswap32(__builtin_bitreverse32(w)) : w;
 }
 
-// Sum over threads of a block (int64); every thread gets the total.
+// Sum over threads of a block (int64), once per kernel; every thread gets the
+// total.
 __device__ __forceinline__ int64_t block_sum(int64_t v, int64_t* red) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -36,7 +38,6 @@ __device__ __forceinline__ int64_t block_sum(int64_t v, int64_t* red) {
   __syncthreads();
   int64_t t = 0;
   for (int i = 0; i < kThreads / 64; ++i) t += red[i];
-  __syncthreads();
   return t;
 }
 
@@ -182,28 +183,26 @@ __device__ __forceinline__ uint32_t row_bits(uint64_t anc, int64_t plen, int64_t
   return low_mask(k) | ((uint32_t)(anc << k) & low_mask(take));
 }
 
-// A thread produces one aligned word of the output (a word that the
-// segment's ends or the capacity cut is stored byte by byte).  Most words lie
-// inside one row's prefix: all ones.  The ancestry rows are read once per
-// workgroup, and there is a thread per word of the capacity, where 8
-// workgroups per segment walked its words with a division and an ancestry
-// read each, and stored bytes wherever a segment starts at an odd one.  us
-// per launch, back to back, before and now (2 words a thread, 4 words):
-//   64 requests x 32 nodes, 4096 tokens          4.0   4.1 (4.5, 5.6)
-//   64 x 16-64 nodes, about 6000 tokens          7.8   5.6 (5.2, 6.0)
-//   1 x 64 nodes, 32768 tokens                  12.3   2.8 (3.0, 3.4)
-//   8 x 8-64 nodes, about 20000 tokens          12.5   3.6 (4.2, 5.2)
-//   128 x 8-64 nodes, about 300 tokens           3.9   4.0 (5.0, 4.9)
+// A thread produces aligned words of the output (a word that the segment's
+// ends or the capacity cut is stored byte by byte).  Most words lie inside one
+// row's prefix: all ones.  The ancestry rows are read once per workgroup, and
+// come in while it sums the earlier segments' sizes.
 __global__ void __launch_bounds__(kThreads) tree_mask_kernel(const dft_mask_args a) {
   __shared__ int64_t red[kThreads / 64];
   __shared__ uint64_t anc[64];
   const int b = blockIdx.y;
   const MaskSeg m = mask_seg(a, b);
-  if ((int)threadIdx.x < m.n) anc[threadIdx.x] = a.anc_bits[m.row0 + threadIdx.x];
+  const int64_t L = m.plen + m.n, nbits = mask_bits(m), nbytes = (nbits + 7) >> 3;
+  // No word falls to this workgroup (at most 3 bytes of the first lie in front
+  // of the segment): said before the sum over the requests ahead.  Workgroup 0
+  // also writes the offsets.
+  if (blockIdx.x > 0 && (int64_t)blockIdx.x * kThreads >= (nbytes + 6) >> 2) return;  // uniform
+  // (the rows come in while the sum runs)
+  const uint64_t mine = (int)threadIdx.x < m.n ? a.anc_bits[m.row0 + threadIdx.x] : 0;
   int64_t part = 0;
   for (int q = threadIdx.x; q < b; q += kThreads) part += (mask_bits(mask_seg(a, q)) + 7) >> 3;
-  const int64_t off = block_sum(part, red);  // (its barriers cover the ancestry rows)
-  const int64_t L = m.plen + m.n, nbits = mask_bits(m), nbytes = (nbits + 7) >> 3;
+  if (threadIdx.x < 64) anc[threadIdx.x] = mine;
+  const int64_t off = block_sum(part, red);  // (its barrier covers the ancestry rows)
   if (a.out_indptr && blockIdx.x == 0 && threadIdx.x == 0) {
     store_indptr(a.out_indptr, a.out_indptr_dtype, b, off);
     if (b + 1 == (int)gridDim.y) store_indptr(a.out_indptr, a.out_indptr_dtype, b + 1, off + nbytes);
@@ -256,12 +255,27 @@ int launch_packbits(const dft_packbits_args* a, hipStream_t stream) {
 }
 
 int launch_tree_mask(const dft_mask_args* a, hipStream_t stream) {
-  // the sizes stay on the device: one thread per word if the requests share
-  // the output's capacity evenly (they stride otherwise), up to a chip's worth
-  // of workgroups
-  const int64_t most = a->batch < 2048 ? 2048 / a->batch : 1;
+  // The sizes stay on the device, so the grid goes by what is known here.  The
+  // capacity bounds the words, one per thread, but is no measure of them where
+  // the buffer is a reserve: no more workgroups for it than kMaskBlocks in all
+  // (one that finds no words costs about 2 ns of launch).  A request may hold
+  // most of the words, and a workgroup alone takes 0.25 us per 256 of them: at
+  // least 8 each up to kMaskWide requests, and 8 kMaskWide in all beyond.  us
+  // per launch, back to back, with 8 workgroups per request that walked its
+  // words by a division and an ancestry read each, with a thread per word of
+  // the capacity up to 2048 workgroups in all, and now (exact buffer / 64 MiB):
+  //   64 requests x 32 nodes, 4096 tokens       3.7    3.8 / 4.6    3.7 / 3.7
+  //   64 x 16-64 nodes, 6000 tokens             6.4    5.2 / 5.4    4.7 / 4.7
+  //   1 x 64 nodes, 32768 tokens               12.2    2.7 / 3.3    2.7 / 2.7
+  //   8 x 64 nodes, 100 tokens                  3.0    3.1 / 4.5    3.1 / 3.2
+  //   128 x 8-64 nodes, 300 tokens              4.0    3.8 / 4.8    3.9 / 3.9
+  //   256 x 8-64 nodes, 2000 tokens             6.8    6.4 / 6.3    6.5 / 6.5
+  //   300 of 100 tokens, one of 64 x 32768     12.4   35.1 /13.1   12.0 /12.0
+  //   2100 of 100 tokens, one of 64 x 32768    33.2   62.3 /62.2   23.3 /23.4
+  const int64_t least = a->batch <= kMaskWide ? 8 : (a->batch < 8 * kMaskWide ? 8 * kMaskWide / a->batch : 1);
+  const int64_t most = a->batch * least < kMaskBlocks ? kMaskBlocks / a->batch : least;
   const int64_t need = (a->out_capacity / a->batch + 4 * kThreads - 1) / (4 * kThreads);
-  const int64_t bx = need < 1 ? 1 : (need > most ? most : need);
+  const int64_t bx = need < least ? least : (need > most ? most : need);
   hipLaunchKernelGGL(tree_mask_kernel, dim3((unsigned)bx, (unsigned)a->batch), dim3(kThreads), 0, stream, *a);
   return hipGetLastError() == hipSuccess ? DFT_OK : DFT_ERR_LAUNCH;
 }

@@ -159,6 +159,36 @@ def test_packbits_alignment(cuda, x_off, out_off, bitorder):
         assert (got[:out_off] == 0xA5).all() and (got[out_off + nbytes:] == 0xA5).all(), n
 
 
+# requests on both sides of each rule of the grid (8 workgroups each, fewer,
+# one), one long request among short ones, a buffer far larger than the masks
+@pytest.mark.parametrize("batch", [1, 95, 97, 1024, 1025, 3000, 8192])
+@pytest.mark.parametrize("reserve", [0, 1 << 22])
+def test_tree_mask_many_requests(cuda, batch, reserve):
+    from dforktree_amd import ops
+    announce(f"tree mask batch={batch} reserve={reserve}")
+    g = np.random.default_rng(batch)
+    sizes = g.integers(0, 6, batch)
+    plens = g.integers(0, 40, batch)
+    sizes[batch // 3], plens[batch // 3] = 64, 20001
+    cu = np.concatenate([[0], np.cumsum(sizes)])
+    bits = g.integers(0, 2 ** 63, int(cu[-1]), dtype=np.int64)
+    segs = []
+    for b in range(batch):
+        n = int(sizes[b])
+        rows = bits[cu[b]:cu[b + 1]].view(np.uint64)
+        anc = (rows[:, None] >> np.arange(n, dtype=np.uint64)[None, :]) & np.uint64(1)
+        segs.append(np.packbits(np.concatenate([np.ones((n, plens[b]), np.uint8), anc.astype(np.uint8)], 1).reshape(-1),
+                                bitorder="little"))
+    want = np.concatenate(segs)
+    buf = torch.full((len(want) + reserve + 16,), 0xA5, dtype=torch.uint8, device=cuda)
+    out, ip = ops.tree_mask_pack(torch.from_numpy(bits).to(cuda), torch.from_numpy(plens).to(cuda),
+                                 cu_seqlens=torch.from_numpy(cu.astype(np.int32)).to(cuda), out=buf[:len(want) + reserve])
+    got = buf.cpu().numpy()
+    assert ip.cpu().numpy().tolist() == [0] + np.cumsum([len(s) for s in segs]).tolist()
+    assert np.array_equal(got[:len(want)], want)
+    assert (got[len(want):] == 0xA5).all()
+
+
 @pytest.mark.parametrize("out_off", [0, 1, 4, 15])
 @pytest.mark.parametrize("bitorder", ["little", "big"])
 def test_tree_mask_alignment(cuda, out_off, bitorder):
