@@ -217,12 +217,12 @@ __global__ void __launch_bounds__(64) tree_conv4_bf16_kernel(const dft_conv_args
 }
 
 // The fast path's main form, for a bf16 conv state and trees of up to 64
-// nodes: a workgroup of 8 waves takes 256 channels of one request and holds
+// nodes: a workgroup of W waves takes 256 channels of one request and holds
 // every column of [conv_state || x] in LDS (and a row of zeros for taps
 // outside it), 512 bytes each.  The token rows are copied in (two per 1 KiB
 // copy) without waiting for the tap columns and are read from memory once
 // instead of once per tap; a lane owns 4 channels, whose weights stay in
-// registers; a wave takes every 8th node of the workgroup's share and reads
+// registers; a wave takes every W-th node of the workgroup's share and reads
 // the next node's columns ahead.
 //
 // A node's window over the slice (iw[n][c][0..2], 1.5 KiB) goes through LDS
@@ -237,9 +237,9 @@ __global__ void __launch_bounds__(64) tree_conv4_bf16_kernel(const dft_conv_args
 // four rows from memory, 37.2 here, 4.5 TB/s; a streaming probe moves 5.2
 // TB/s at this mix of reads and writes.  The same rows in cache: 42.0 -> 32.8.
 // Batch 4: 8.2 -> 5.6, batch 1 (plugin step, 24 layers): 354 -> 334, and 330
-// -> 318 once no load of the prologue waited for another.  4 waves took 1.2 us
-// longer, 16 4 us.
-constexpr int kConvNodes = 64, kConvSlice = 256, kConvWaves = 8;
+// -> 318 once no load of the prologue waited for another.  8 waves; 4 took 1.2
+// us longer, 16 4 us (small trees: launch_conv4_rows).
+constexpr int kConvNodes = 64, kConvSlice = 256;
 
 // rows of the workgroup's LDS: zeros, 3 state columns, the tokens (an odd
 // count's last copy fills one more)
@@ -267,9 +267,8 @@ __device__ __forceinline__ void tap_rows(const uint16_t* rows, const int* taps, 
   r[3] = *reinterpret_cast<const uint2*>(base + t.w);
 }
 
-template <bool CIDX64>
-__global__ void __launch_bounds__(64 * kConvWaves) tree_conv4_rows_kernel(const dft_conv_args p, int cblocks,
-                                                                          int splits) {
+template <bool CIDX64, int W>
+__global__ void __launch_bounds__(64 * W) tree_conv4_rows_kernel(const dft_conv_args p, int cblocks, int splits) {
   // Every load of the prologue goes out before anything waits for one of
   // them: read where they are used, the tap columns were waited for (and with
   // them the row copies ahead of them) before the weights and the state were
@@ -300,7 +299,7 @@ __global__ void __launch_bounds__(64 * kConvWaves) tree_conv4_rows_kernel(const 
     // (channels past the last read channel 0 of the slice instead)
     const uint16_t* xb = static_cast<const uint16_t*>(p.x) + (int64_t)b * p.x_req_stride + cbase;
     const int c8 = 8 * (lane & 31), half = lane >> 5;
-    for (int r = 2 * wave; r < N; r += 2 * kConvWaves)
+    for (int r = 2 * wave; r < N; r += 2 * W)
       __builtin_amdgcn_global_load_lds(xb + min(r + half, N - 1) * p.x_node_stride + (c8 < nch ? c8 : 0),
                                        (__attribute__((address_space(3))) void*)(rows + (4 + r) * kConvSlice), 16, 0, 0);
   }
@@ -314,11 +313,17 @@ __global__ void __launch_bounds__(64 * kConvWaves) tree_conv4_rows_kernel(const 
   const u32x4* wp = reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(p.weight) +
                                                    (int64_t)(cbase + (active ? c0 : 0)) * 4);
   const u32x4 wraw[2] = {wp[0], wp[1]};
-  // one channel of the state per thread
-  const int chan = min(tid, nch - 1);
+  // the state: a channel per thread, or every 64 W-th
+  constexpr int SC = W < 4 ? 4 / W : 1;
   const uint16_t* cs = static_cast<const uint16_t*>(p.conv_state) + (slot_raw < 0 ? 0 : slot_raw) * p.cs_slot_stride +
-                       (int64_t)(cbase + chan) * p.cs_chan_stride;
-  const uint16_t state[3] = {cs[0], cs[p.cs_col_stride], cs[2 * p.cs_col_stride]};
+                       (int64_t)cbase * p.cs_chan_stride;
+  uint16_t state[SC][3];
+#pragma unroll
+  for (int q = 0; q < SC; ++q) {
+    const uint16_t* col = cs + (int64_t)min(tid + 64 * W * q, nch - 1) * p.cs_chan_stride;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) state[q][j] = col[j * p.cs_col_stride];
+  }
   __builtin_amdgcn_sched_barrier(0);
 
   if (tid < 4 * N) {
@@ -333,9 +338,13 @@ __global__ void __launch_bounds__(64 * kConvWaves) tree_conv4_rows_kernel(const 
       w[8 * q + 2 * e] = __uint_as_float(wraw[q][e] << 16);
       w[8 * q + 2 * e + 1] = __uint_as_float(wraw[q][e] & 0xffff0000u);
     }
-  if (tid < nch) {
 #pragma unroll
-    for (int j = 0; j < 3; ++j) rows[(1 + j) * kConvSlice + tid] = state[j];
+  for (int q = 0; q < SC; ++q) {
+    const int c = tid + 64 * W * q;
+    if (c < nch) {
+#pragma unroll
+      for (int j = 0; j < 3; ++j) rows[(1 + j) * kConvSlice + c] = state[q][j];
+    }
   }
   float bias[4] = {0.f, 0.f, 0.f, 0.f};
   if (p.bias) {  // uniform
@@ -354,9 +363,9 @@ __global__ void __launch_bounds__(64 * kConvWaves) tree_conv4_rows_kernel(const 
   int n = split * share + wave;
   uint2 next[4] = {};
   if (n < n_end) tap_rows(rows, taps, n, lane, next);
-  for (; n < n_end; n += kConvWaves) {
+  for (; n < n_end; n += W) {
     const uint2 r[4] = {next[0], next[1], next[2], next[3]};
-    if (n + kConvWaves < n_end) tap_rows(rows, taps, n + kConvWaves, lane, next);
+    if (n + W < n_end) tap_rows(rows, taps, n + W, lane, next);
     float acc[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc[e] = bias[e];
@@ -416,21 +425,44 @@ static bool conv4_bf16_ok(const dft_conv_args* a) {
 // A launch of few (request, slice) pairs divides each pair's nodes over
 // several workgroups, which each copy all rows in, until there is one per CU
 // or a wave has one node (batch 1: 334 us per plugin step, 375 undivided).
-// More nodes than the LDS rows hold, or a conv state of another type, take
-// the per-node kernel.
+template <int W>
+static void launch_rows_kernel(const dft_conv_args* a, int cblocks, int64_t pairs8, hipStream_t stream) {
+  int splits = 1;
+  while (splits * W < a->n_nodes && pairs8 * 8 * splits < 256) splits *= 2;
+  const size_t lds = 2 * kConvSlice * (size_t)conv_rows(a->n_nodes) + 16 * a->n_nodes + 6 * kConvSlice * W;
+  const dim3 grid((unsigned)(pairs8 * 8 * splits)), block(64 * W);
+  if (a->cidx_dtype == DFT_I64)
+    hipLaunchKernelGGL((tree_conv4_rows_kernel<true, W>), grid, block, lds, stream, *a, cblocks, splits);
+  else
+    hipLaunchKernelGGL((tree_conv4_rows_kernel<false, W>), grid, block, lds, stream, *a, cblocks, splits);
+}
+
+// 8 waves per workgroup, or fewer where they would have no node to take: a
+// launch of many pairs is then bound by the waves it starts.  Beyond 4 nodes a
+// launch below kConvPairs is not, and the 8 share the copies.  us for 8192
+// channels (32 pairs per request), without and with the window, 8 waves / fewer
+// (in brackets a one-wave workgroup per node, the kernel above):
+//   batch 64, 1 node    7.3 / 4.5   [5.2]    7.8 / 5.0   [5.9]
+//   batch 64, 3         9.0 / 6.4   [7.9]    9.9 / 7.3   [9.7]
+//   batch 512, 1       38.9 / 17.1 [18.4]   39.1 / 18.0 [20.8]
+//   batch 512, 5       56.8 / 37.9 [47.4]   61.4 / 44.9 [58.4]
+//   batch 64, 12       13.4 / 11.0 [17.2]   14.5 / 13.0 [20.7]
+//   batch 8, 8          3.9 / 4.0   [5.2]    4.3 / 4.6   [5.9]   (8 waves taken)
+//   batch 8, 3          3.7 / 3.6   [4.6]    3.9 / 3.8   [5.1]
+// More nodes than the LDS rows hold, or a conv state of another type, take the
+// per-node kernel.
+constexpr int64_t kConvPairs = 1024;
 static bool launch_conv4_rows(const dft_conv_args* a, hipStream_t stream) {
   if (a->cs_dtype != DFT_BF16 || a->n_nodes > kConvNodes) return false;
   const int cblocks = (a->channels + kConvSlice - 1) / kConvSlice;
   const int64_t pairs8 = ((int64_t)a->batch * cblocks + 7) / 8;
-  int splits = 1;
-  while (splits * kConvWaves < a->n_nodes && pairs8 * 8 * splits < 256) splits *= 2;
-  if (pairs8 * 8 * splits > (int64_t)0xffffffffll / (64 * kConvWaves)) return false;  // work-items in 32 bits
-  const size_t lds = 2 * kConvSlice * (size_t)conv_rows(a->n_nodes) + 16 * a->n_nodes + 6 * kConvSlice * kConvWaves;
-  const dim3 grid((unsigned)(pairs8 * 8 * splits)), block(64 * kConvWaves);
-  if (a->cidx_dtype == DFT_I64)
-    hipLaunchKernelGGL(tree_conv4_rows_kernel<true>, grid, block, lds, stream, *a, cblocks, splits);
+  if (pairs8 * 8 > (int64_t)0xffffffffll / (64 * 8)) return false;  // work-items in 32 bits (undivided: 256 pairs or more)
+  if (a->n_nodes <= 2)
+    launch_rows_kernel<2>(a, cblocks, pairs8, stream);
+  else if (a->n_nodes <= 4 || (a->n_nodes <= 12 && pairs8 * 8 >= kConvPairs))
+    launch_rows_kernel<4>(a, cblocks, pairs8, stream);
   else
-    hipLaunchKernelGGL(tree_conv4_rows_kernel<false>, grid, block, lds, stream, *a, cblocks, splits);
+    launch_rows_kernel<8>(a, cblocks, pairs8, stream);
   return true;
 }
 

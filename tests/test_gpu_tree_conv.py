@@ -364,11 +364,13 @@ def test_anc_pack_matches_oracle_bits(cuda, n):
 
 # nodes on both sides of a wave's and a workgroup's share and of the LDS rows'
 # limit, slices cut at 8 channels, taps outside [conv_state || x], each index
-# width; a float conv state takes the per-node kernel
+# width, small trees in small launches and in large ones (of 1024 slices on);
+# a float conv state takes the per-node kernel
 @pytest.mark.parametrize("cs_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("B,N,C", [(1, 1, 8), (1, 2, 256), (2, 7, 248), (1, 8, 264), (3, 9, 1000), (9, 16, 512),
                                    (1, 31, 2048), (2, 33, 776), (70, 5, 1024), (1, 63, 264), (5, 64, 520),
-                                   (2, 65, 256)])
+                                   (2, 65, 256), (3, 1, 520), (5, 3, 264), (2, 4, 776), (1, 5, 8), (600, 2, 264),
+                                   (350, 3, 520), (255, 5, 1024), (257, 5, 1000), (1030, 12, 8), (1030, 13, 256)])
 def test_conv_slices(cuda, B, N, C, cs_dtype):
     from dforktree_amd import ops
     announce(f"conv slices B={B} N={N} C={C} {cs_dtype}")
