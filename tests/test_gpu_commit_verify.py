@@ -171,16 +171,18 @@ def test_commit_verify_packed_ragged_per_khead(cuda, path_dtype):
     _check_chain(batch1, batch2, pool, o2, aux2, walks, empty, per_khead=True)
 
 
-def test_commit_verify_size_order(cuda):
+@pytest.mark.parametrize("hk,hv", [(2, 4), (3, 3)], ids=["mixed_kernel", "two_kernels"])
+def test_commit_verify_size_order(cuda, hk, hv):
     """Packed trees on both sides of 32 nodes in both steps, recomputed
     values and raw keys: the fused launch reading size-order records commits
-    and verifies bit for bit as the launch without them."""
+    and verifies bit for bit as the launch without them, as the mixed-width
+    kernel and (an odd head count) as two kernels."""
     from dforktree_amd import synth
-    announce("commit->verify with size-order records")
+    announce(f"commit->verify with size-order records hk={hk} hv={hv}")
     sizes1, kinds = [40, 9, 64, 17, 33, 1, 50, 20], ["random", "chain", "bushy", "random"] * 2
     sizes2 = [12, 64, 30, 1, 50, 20, 33, 64]
-    batch1 = synth.make_batch(52, 0, sizes1, hk=2, hv=4, kinds=kinds)
-    batch2 = synth.make_batch(53, 0, sizes2, hk=2, hv=4, kinds=kinds)
+    batch1 = synth.make_batch(52, 0, sizes1, hk=hk, hv=hv, kinds=kinds)
+    batch2 = synth.make_batch(53, 0, sizes2, hk=hk, hv=hv, kinds=kinds)
     runs = [_run_chain(cuda, batch1, batch2, per_khead=True, packed=True, empty=(3,), shorten=(6,), raw_keys=True,
                        raw_values=True, ordered=ordered) for ordered in (False, True)]
     (pa, oa, auxa, walks), (pb, ob, auxb, _) = runs

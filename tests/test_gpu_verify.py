@@ -100,12 +100,14 @@ def test_verify_batched_uniform_bits(cuda):
     check_against_oracle(batch, *run_gpu(batch, cuda, use_bits=True))
 
 
-@pytest.mark.parametrize("hk,hv,records", [(2, 4, False), (2, 4, True), (2, 2, True), (1, 4, True), (2, 8, True)])
+@pytest.mark.parametrize("hk,hv,records", [(2, 4, False), (2, 4, True), (2, 2, True), (1, 4, True), (2, 8, True),
+                                           (3, 3, False), (3, 3, True), (1, 17, False), (1, 17, True)])
 def test_verify_packed_ragged(cuda, hk, hv, records):
-    """Packed varlen rows with cu_seqlens, sizes 1..64: two kernels without
-    size-order records, the mixed-width kernel with them, whose v-head pairs
-    (2j, 2j + 1) span one k-head (R = 2), two k-heads (R = 1) or half of one
-    (R = 4)."""
+    """Packed varlen rows with cu_seqlens, sizes 1..64: the mixed-width kernel
+    without and with size-order records, its v-head pairs (2j, 2j + 1)
+    spanning one k-head (R = 2), two k-heads (R = 1) or half of one (R = 4);
+    with an odd head count the column-split pair of kernels (24 items) and
+    the unsplit pair (136 items)."""
     from dforktree_amd import synth
     announce(f"verify packed ragged hk={hk} hv={hv} records={records}")
     sizes, kinds = [8, 64, 17, 1, 33, 64, 40, 9], ["chain", "random", "bushy", "random", "chain", "bushy",
@@ -114,16 +116,20 @@ def test_verify_packed_ragged(cuda, hk, hv, records):
     check_against_oracle(batch, *run_gpu(batch, cuda, packed=True, records=records))
 
 
-@pytest.mark.parametrize("records", [False, True], ids=["two_kernels", "mixed_kernel"])
-def test_verify_split_order_empty_requests_and_slots(cuda, records):
-    """A launch split by tree size, as two kernels or (with size-order
-    records) as the mixed-width kernel: empty requests between the others,
-    permuted state slots with a -1 (read from slot 0), trees on both sides of
-    32 nodes.  Every request matches the oracle and reports status 0."""
+@pytest.mark.parametrize("hk,hv,records", [(2, 4, False), (2, 4, True), (3, 3, False), (3, 3, True), (1, 13, False),
+                                           (1, 13, True)],
+                         ids=["mixed_kernel_no_records", "mixed_kernel", "column_split", "column_split_records",
+                              "two_kernels", "two_kernels_records"])
+def test_verify_split_order_empty_requests_and_slots(cuda, hk, hv, records):
+    """A launch split by tree size, as the mixed-width kernel or (odd head
+    counts) as two kernels, column-split (36 items) or not (156), each without
+    and with size-order records: empty requests between the others, permuted
+    state slots with a -1 (read from slot 0), trees on both sides of 32 nodes.
+    Every request matches the oracle and reports status 0."""
     from dforktree_amd import ops, synth
-    announce(f"verify split order: empty requests, slots, records={records}")
+    announce(f"verify split order: empty requests, slots, hk={hk} hv={hv} records={records}")
     sizes = [40, 12, 64, 33, 9, 17, 64, 1, 48]
-    batch = synth.make_batch(23, 0, sizes, hk=2, hv=4, kinds=["random", "chain", "bushy"] * 3)
+    batch = synth.make_batch(23, 0, sizes, hk=hk, hv=hv, kinds=["random", "chain", "bushy"] * 3)
     empty_at = [1, 5, 9]  # positions of the empty requests in the launch
     order = []            # launch position -> index into sizes (None: empty)
     it = iter(range(len(sizes)))
@@ -132,20 +138,20 @@ def test_verify_split_order_empty_requests_and_slots(cuda, records):
     lens = [0 if r is None else sizes[r] for r in order]
     cu = torch.zeros(len(order) + 1, dtype=torch.int32)
     cu[1:] = torch.cumsum(torch.tensor(lens, dtype=torch.int32), 0)
-    pool = torch.randn(len(order) + 1, 4, 128, 128) * 0.02
+    pool = torch.randn(len(order) + 1, hv, 128, 128) * 0.02
     slots = torch.randperm(len(order) + 1)[:len(order)].to(torch.int32)
     slots[3] = -1
     batch.state = torch.stack([pool[max(int(slots[p]), 0)] for p, r in enumerate(order) if r is not None])
     g = batch.to(cuda)
     rows = g.y.shape[0]
     ts = ops.tree_struct(g.parent, 4, cu_seqlens=g.cu_seqlens, n_nodes=64, batch=batch.batch, want=("anc_bits",))
-    aux_k = torch.zeros(4, rows, 128, device=cuda)
-    aux_v = torch.zeros(4, rows, 128, device=cuda)
-    aux_g = torch.zeros(4, rows, device=cuda)
+    aux_k = torch.zeros(hv, rows, 128, device=cuda)
+    aux_v = torch.zeros(hv, rows, 128, device=cuda)
+    aux_g = torch.zeros(hv, rows, device=cuda)
     status = torch.full((len(order),), -5, device=cuda, dtype=torch.int32)
     cu_d = cu.to(cuda)
     so = ops.size_order(cu_d, 64) if records else None
-    o = ops.tree_verify(g.y, g.a, g.b, g.A_log, g.dt_bias, pool.to(cuda).transpose(-1, -2), hk=2, hv=4,
+    o = ops.tree_verify(g.y, g.a, g.b, g.A_log, g.dt_bias, pool.to(cuda).transpose(-1, -2), hk=hk, hv=hv,
                         anc_bits=ts["anc_bits"], cu_seqlens=cu_d, n_nodes=64, batch=len(order),
                         state_indices=slots.to(cuda), aux_k=aux_k, aux_v=aux_v, aux_g=aux_g, status=status,
                         size_order=so)
@@ -154,16 +160,17 @@ def test_verify_split_order_empty_requests_and_slots(cuda, records):
     check_against_oracle(batch, o, aux_k, aux_v, aux_g)
 
 
+@pytest.mark.parametrize("records", [True, False])
 @pytest.mark.parametrize("sizes", [[5, 32, 17, 1, 30, 9], [33, 64, 40, 48]], ids=["all_small", "all_large"])
-def test_verify_mixed_kernel_one_class(cuda, sizes):
-    """Size-order records of a batch whose trees are all on one side of 32
-    nodes (launched at n_nodes 64): the mixed-width kernel then runs only
-    v-head pairs on the 32-wide body, or only 64-wide items.  Against the
-    oracle."""
+def test_verify_mixed_kernel_one_class(cuda, sizes, records):
+    """A batch whose trees are all on one side of 32 nodes (launched at
+    n_nodes 64), with size-order records and without: the mixed-width kernel
+    then runs only v-head pairs on the 32-wide body, or only 64-wide items.
+    Against the oracle."""
     from dforktree_amd import synth
-    announce(f"verify mixed kernel, one size class: {sizes}")
+    announce(f"verify mixed kernel, one size class: {sizes} records={records}")
     batch = synth.make_batch(31, 0, sizes, hk=2, hv=4, kinds=["random", "chain", "bushy"] * 2)
-    check_against_oracle(batch, *run_gpu(batch, cuda, packed=True, records=True, n_nodes=64))
+    check_against_oracle(batch, *run_gpu(batch, cuda, packed=True, records=records, n_nodes=64))
 
 
 def size_order_records(cu, n_nodes):
@@ -391,13 +398,16 @@ def test_verify_kmajor_state_64_wide_split(cuda):
     check_against_oracle(batch, o, k, v, g)
 
 
+@pytest.mark.parametrize("hk,hv", [(2, 4), (3, 3), (3, 33)], ids=["mixed_kernel", "column_split", "one_workgroup"])
 @pytest.mark.parametrize("o_dtype", [torch.bfloat16, torch.float32])
-def test_verify_64_wide_output_forms(cuda, o_dtype):
-    """The 64-wide kernel with staged bf16 output (o staged in X) and with
-    direct fp32 stores, trees of 33-64 nodes only."""
+def test_verify_64_wide_output_forms(cuda, o_dtype, hk, hv):
+    """The 64-wide body with staged bf16 output (o staged in X) and with
+    direct fp32 stores, trees of 33-64 nodes only, in the mixed-width kernel
+    and (odd head counts) the 64-wide kernel, column-split (12 items) or not
+    (132)."""
     from dforktree_amd import synth
-    announce(f"verify 64-wide {o_dtype}")
-    batch = synth.make_batch(19, 0, [64, 48, 33, 57], hk=2, hv=4, kinds=["random", "chain", "bushy", "random"])
+    announce(f"verify 64-wide {o_dtype} hk={hk} hv={hv}")
+    batch = synth.make_batch(19, 0, [64, 48, 33, 57], hk=hk, hv=hv, kinds=["random", "chain", "bushy", "random"])
     o, k, v, g = run_gpu(batch, cuda, o_dtype=o_dtype, packed=True)
     check_against_oracle(batch, o, k, v, g, o_bf16=(o_dtype == torch.bfloat16))
 
@@ -406,9 +416,10 @@ def test_verify_64_wide_output_forms(cuda, o_dtype):
 def test_verify_64_wide_column_split(cuda, case):
     """Launches over 32 nodes with at most 128 (request, v-head) items run
     each item on two workgroups (value columns split, state k halves split
-    over wave pairs): batch 1 and 4 at full width (32 v-heads) take that
-    form, batch 5 (160 items) the one-workgroup kernel.  fp32 output is held
-    to 5e-5, as the one-workgroup kernel is."""
+    over wave pairs) unless they are packed with an even head count (the
+    mixed-width kernel): batch 1 at full width (32 v-heads) and a packed
+    batch 4 with 31 take that form, batch 5 (160 items) the one-workgroup
+    kernel.  fp32 output is held to 5e-5, as the one-workgroup kernel is."""
     from dforktree_amd import synth
     announce(f"verify 64-wide column split {case}")
     if case == "b1_fp32_dense":
@@ -419,8 +430,8 @@ def test_verify_64_wide_column_split(cuda, case):
         assert rel_l2(np32(v), ref["vn"]) <= 5e-5
         check_against_oracle(batch, o, k, v, g, o_bf16=False)
     elif case == "b4_packed_slots":
-        batch = synth.make_batch(22, 0, [64, 40, 9, 33], hk=16, hv=32, kinds=["chain", "random", "bushy", "random"])
-        pool = torch.randn(6, 32, 128, 128) * 0.02
+        batch = synth.make_batch(22, 0, [64, 40, 9, 33], hk=31, hv=31, kinds=["chain", "random", "bushy", "random"])
+        pool = torch.randn(6, 31, 128, 128) * 0.02
         slots = torch.tensor([5, 0, -1, 2], dtype=torch.int32)
         batch.state = pool[slots.clamp(min=0).long()]
         o, k, v, g = run_gpu(batch, cuda, packed=True, state=pool.to(cuda), state_indices=slots.to(cuda))
