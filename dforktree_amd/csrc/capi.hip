@@ -27,6 +27,10 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 // workgroups of `threads` threads.
 constexpr int64_t max_blocks(int threads) { return (int64_t)0xffffffffll / threads; }
 
+// The tree-structure and ancestry-pack entry points' largest batch: a wave per
+// request in one grid, though their workgroups stride over further requests.
+constexpr int64_t kMaxRequests = 4 * max_blocks(256);
+
 // Checks shared by the verify entry points: DFT_OK to launch, DFT_ERR_* to
 // refuse, or -1 when there is nothing to do.  commit_only: a launch of the
 // fused entry with n_nodes 0, which commits the pending paths and verifies
@@ -63,7 +67,7 @@ int tree_status(const dft_tree_args* a) {
   if (a->batch < 0 || a->n_nodes < 0 || a->n_nodes > 64) return DFT_ERR_INVALID;
   if (a->kc < 0 || a->kc > 16) return DFT_ERR_UNSUPPORTED;
   if (a->batch == 0) return -1;
-  if (((int64_t)a->batch + 3) / 4 > max_blocks(256)) return DFT_ERR_UNSUPPORTED;
+  if (a->batch > kMaxRequests) return DFT_ERR_UNSUPPORTED;
   if (!a->parent || !index_tag(a->parent_dtype)) return DFT_ERR_INVALID;
   if (a->depth && !index_tag(a->depth_dtype)) return DFT_ERR_INVALID;
   if (a->cidx && (!index_tag(a->cidx_dtype) || a->kc < 1)) return DFT_ERR_INVALID;
@@ -192,7 +196,7 @@ int dft_anc_pack(const dft_anc_pack_args* a, void* stream) {
   if (!a) return DFT_ERR_INVALID;
   if (a->batch < 0 || a->n_nodes < 0 || a->n_nodes > 64) return DFT_ERR_INVALID;
   if (a->batch == 0 || a->n_nodes == 0) return DFT_OK;
-  if (((int64_t)a->batch + 3) / 4 > max_blocks(256)) return DFT_ERR_UNSUPPORTED;
+  if (a->batch > kMaxRequests) return DFT_ERR_UNSUPPORTED;
   if (!a->anc || !a->anc_bits) return DFT_ERR_INVALID;
   return dft::launch_anc_pack(a, static_cast<hipStream_t>(stream));
 }

@@ -370,8 +370,9 @@ __device__ __forceinline__ float quad_bcast(float x) {
 // row m: one aligned 16-byte read, issued kAhead steps before its use).
 // A's entries at and above the diagonal are zero (the tile is masked to
 // strict ancestors, which precede a node), so rows i <= m are left as they
-// are and each element sees the same fused multiply-adds in the same order
-// as in solve_block16: the result is bit-identical.  A step is one move and
+// are (x_m is finite for finite rows: |A| <= 1) and each element sees the same
+// fused multiply-adds in the same order as in solve_block16: the result is
+// bit-identical.  A step is one move and
 // four multiply-adds on the chain instead of up to 15, and one 16-byte read.
 // Writes X_bb to x (pitch LDA) at (base, base).
 template <int LDA, int kAhead>
@@ -979,8 +980,8 @@ __device__ __forceinline__ void path_values(const Pending& pd, const float* pkey
     const bool ok = (pd.vmask >> ip) & 1u;
 #pragma unroll
     for (int t = 0; t < TT; ++t) {
-      const uint16_t vb = VLDS ? reinterpret_cast<const uint16_t*>(pkey)[qkv_at(16 + ip, col0 + Waves<NWC>::CW * wave + 16 * t + n16)]
-                               : vr[e][t];
+      const int col = col0 + Waves<NWC>::CW * wave + 16 * t + n16;
+      const uint16_t vb = VLDS ? reinterpret_cast<const uint16_t*>(pkey)[qkv_at(16 + ip, col)] : vr[e][t];
       w[t][e] = ok ? bp * (bf16_bits_to_f32(vb) - ep * w[t][e]) : 0.f;
     }
   }
@@ -2751,16 +2752,34 @@ int launch_size_order(const int32_t* cu_seqlens, int batch, int n_nodes, int32_t
 }
 
 // Whether a launch split by tree size runs as one mixed-width launch: with
-// size-order records, and without them in small launches, where the second
-// kernel's start and the emptier chip cost more than the workgroups that
-// exit between the others.  us per 8 layers of 8-64 nodes, 32 heads, two
+// size-order records, and without them in small launches (up to kMixedItems
+// items), where the second kernel's start and the emptier chip cost more than
+// the workgroups that exit between the others.  us per layer at 32 heads, two
 // kernels / one:
-//   verify + commit, records     batch 2 174 / 128, 8 170 / 163, 32 428 / 418
-//   fused (raw rows), records    batch 2 234 / 150, 8 277 / 170, 48 562 / 531
-//   fused (saves), records       batch 16 291 / 241, 32 415 / 372, 48 611 / 542
-//   fused (raw rows), none       batch 2 232 / 150, 24 401 / 379, 48 619 / 668
-//   fused (saves), none          batch 16 349 / 243, 32 469 / 451, 48 621 / 649
-// (the forms other than raw rows spill 6-8 registers in the mixed kernel).
+//                                     8-64 nodes     3-36 nodes     33-64 nodes
+//   verify, records       batch 16   21.0 /  20.3   18.5 /  18.3   22.1 /  21.4
+//                         batch 64   62.7 /  61.7   48.4 /  48.0   75.6 /  74.1
+//   verify, none          batch 4    19.4 /  13.9   19.1 /  13.2   14.7 /  13.9  (two column-split kernels)
+//                         batch 16   27.1 /  21.5   27.1 /  19.3   22.7 /  21.0
+//                         batch 24   36.1 /  30.5   31.4 /  27.1   34.2 /  31.1
+//   fused raw, records    batch 8    35.1 /  21.6   35.9 /  23.8   22.9 /  21.3
+//                         batch 64   93.4 /  88.4   77.9 /  74.2   98.4 /  98.8
+//                         batch 128 167.6 / 165.0  129.0 / 132.5  182.9 / 185.0
+//   fused raw, none       batch 22   46.8 /  43.4   47.1 /  43.1   41.3 /  40.7
+//                         batch 24   53.1 /  44.9   47.5 /  50.5   43.8 /  42.7
+//   fused saves, records  batch 64   97.0 /  91.7   80.8 /  77.2  102.2 /  99.6
+//   fused saves, none     batch 22   46.0 /  42.9   45.9 /  42.0   47.1 /  43.0
+//                         batch 24   52.7 /  47.4   46.7 /  48.4   48.7 /  45.8
+//                         batch 48 (raw / saves, 8-64)   619 / 668 and 621 / 649 per 8 layers
+// (the fused forms other than raw rows spill 6-8 registers in the mixed
+// kernel).  One kernel loses in places, by the share of a last generation: at
+// 768 items without records (above; saves of 20-40 nodes 45.5 / 50.5), and
+// with records where few large trees stand among many small ones in several
+// generations (raw rows, 8 of 33-64 among 3-32: batch 64 76.0 / 77.2, 96 99.1
+// / 105.2, 128 125.8 / 130.8).  The sizes are the device's: a rule on the batch
+// alone would cost the ranges of sizes more than it gives those (48 ranges
+// from 1, 8 or 16 up to 36 ... 64, raw rows with records, batch 96 and 128:
+// 2.5% less as one kernel, five of them up to 1.7% more).
 constexpr int64_t kMixedItems = 768;
 static bool mixed_launch(const dft_verify_args* a, bool split) {
   return split && a->hv % 2 == 0 && (a->size_order || (int64_t)a->batch * a->hv <= kMixedItems);

@@ -155,11 +155,14 @@ typedef struct dft_verify_args {
   /* DFT_ABI_VERSION 4 (appended).  Optional: the packed batch's requests
    * ordered by size class, as dft_size_order writes them from the same
    * cu_seqlens and n_nodes.  A packed launch split by tree size (n_nodes >
-   * 32) then gives each of its two kernels its own requests first, read from
-   * the records: the workgroups past a class's count exit at the end of the
+   * 32) then takes the requests from the records, the large trees first: as
+   * one kernel for both classes if hv is even (and the state has k stride 1
+   * and 16-byte aligned rows), else as two kernels that each take their own
+   * class first.  The workgroups past the last request exit at the end of the
    * grid, in the slots its last generation leaves idle, instead of among the
-   * work (128 requests of 8-64 nodes: 115.8 -> 113.5 us per layer).  Ignored
-   * by unsplit launches; must not be written while the launch runs. */
+   * work (128 requests of 8-64 nodes: 115.8 us per layer without records,
+   * 113.5 as two kernels, 111.7 as one).  Ignored by unsplit launches; must
+   * not be written while the launch runs. */
   const int32_t* size_order;
 } dft_verify_args;
 
@@ -174,8 +177,7 @@ DFT_API int dft_tree_verify(const dft_verify_args* args, void* stream);
  * reference (its launches are per tree size, tree_kernels.py:193-208): for
  * callers of packed ragged batches, once per step and shared by all layers.
  * A launch whose n_nodes or batch differs from the header's ignores the
- * records (each kernel then takes the requests in block order, as without
- * them); records written from other cu_seqlens of the same n_nodes and
+ * records (the requests are then taken in block order, as without them); records written from other cu_seqlens of the same n_nodes and
  * batch are not detected here.
  * DFT_ERR_INVALID for batch < 0, n_nodes outside 1..64 or a null pointer. */
 DFT_API int dft_size_order(const int32_t* cu_seqlens, int32_t batch, int32_t n_nodes, int32_t* order,
