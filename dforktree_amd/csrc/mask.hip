@@ -19,7 +19,7 @@ namespace dft {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kBlocksPerSegment = 8;  // workgroups per packbits segment (grid-stride over its words)
+constexpr int kBlocksPerSegment = 8, kSegmentBlocks = 6144;  // launch_packbits
 constexpr int64_t kMaskBlocks = 768, kMaskWide = 1024;  // launch_tree_mask
 
 __device__ __forceinline__ uint32_t low_mask(int bits) { return bits >= 32 ? 0xffffffffu : ((1u << bits) - 1u); }
@@ -103,10 +103,11 @@ typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 // A thread packs the 32 elements of one aligned word of the output.  They
 // come as whole dwords (two 16-byte loads; where the elements start inside a
 // dword one more, and the bytes are shifted into place: every dword read
-// holds at least one of the elements), 8 elements at a time only in a word
-// that the segment's ends cut.  Read one by one, the 32 elements were 32
-// loads of one byte, 32 apart between lanes: 6.9 us per launch for a 64 x
-// 32795 mask (2.1 MB), now 2.6 us.
+// holds at least one of the elements), one by one only in a word that the
+// segment's ends cut (16 loads at once: 500 segments of 77 elements 11.6 ->
+// 9.2 us; 32 at once take 76 registers and 6% more on a large mask).  Read one
+// by one, the 32 elements of every word were 32 loads of one byte, 32 apart
+// between lanes: 6.9 us per launch for a 64 x 32795 mask (2.1 MB), now 2.6.
 __global__ void __launch_bounds__(kThreads) packbits_kernel(const dft_packbits_args a) {
   __shared__ int64_t red[kThreads / 64];
   const int s = blockIdx.y;
@@ -140,10 +141,17 @@ __global__ void __launch_bounds__(kThreads) packbits_kernel(const dft_packbits_a
       }
       const uint32_t el[8] = {d[0], d[1], d[2], d[3], d[4], d[5], d[6], d[7]};
       word = pack32(el);
-    } else {
-#pragma unroll 8
-      for (int t = 0; t < 32; ++t)
-        if (e0 + t >= 0 && e0 + t < len && x[e0 + t] != 0) word |= 1u << t;
+    } else {  // elements lo .. hi of the word: clamped, always valid addresses, 16 loads at once
+      const int lo = e0 < 0 ? (int)-e0 : 0, hi = len - e0 < 32 ? (int)(len - e0) - 1 : 31;
+#pragma unroll 1
+      for (int h = 0; h < 32; h += 16) {
+        uint8_t v[16];
+#pragma unroll
+        for (int t = 0; t < 16; ++t) v[t] = x[e0 + min(max(h + t, lo), hi)];
+#pragma unroll
+        for (int t = 0; t < 16; ++t) word |= (uint32_t)(v[t] != 0) << (h + t);
+      }
+      word &= low_mask(hi + 1) & ~low_mask(lo);
     }
     ok &= store_word(a.out, a.out_capacity, off, nbytes, j, to_order(word, a.bit_order));
   }
@@ -244,8 +252,17 @@ __global__ void __launch_bounds__(kThreads) tree_mask_kernel(const dft_mask_args
 
 int launch_packbits(const dft_packbits_args* a, hipStream_t stream) {
   const int segs = a->indptr ? a->n_segments : 1;
-  // one segment of known length: enough workgroups to cover it once
-  int bx = kBlocksPerSegment;
+  // Segments (their sizes stay on the device): 8 workgroups each that stride
+  // over its words, fewer where there are so many that starting them is the
+  // launch's time.  us with 8 for each and the cut words' elements one after
+  // another / now (in brackets the form that read every word so):
+  //   1000 segments of 77 elements         19.0 /  11.6   [17.5]
+  //   3000                                 58.4 /  17.8   [54.5]
+  //   9000                                273.8 /  41.2  [264.1]
+  //   3000, one of them of 2^21            59.1 /  54.0  [145.3]
+  // One segment of known length: enough workgroups to cover it once.
+  int bx = segs <= kSegmentBlocks / kBlocksPerSegment ? kBlocksPerSegment
+                                                      : (segs < kSegmentBlocks ? kSegmentBlocks / segs : 1);
   if (!a->indptr) {
     const int64_t words = ((a->n + 31) >> 5) + 1, need = (words + kThreads - 1) / kThreads;  // (+ 1: an unaligned out)
     bx = (int)(need < 1 ? 1 : (need > 4096 ? 4096 : need));

@@ -41,6 +41,28 @@ def test_segment_packbits(cuda):
         assert new.cpu().numpy().tolist() == want_ip.tolist()
 
 
+# segments on both sides of each rule of the grid (8 workgroups each, fewer,
+# one), short ones that the output's words cut at both ends, one long one
+@pytest.mark.parametrize("segs", [1, 768, 769, 3000, 6145])
+@pytest.mark.parametrize("bitorder", ["little", "big"])
+def test_segment_packbits_many(cuda, segs, bitorder):
+    from dforktree_amd import ops
+    announce(f"segment_packbits {segs} segments {bitorder}")
+    g = np.random.default_rng(segs)
+    lens = g.integers(0, 90, segs)
+    lens[segs // 2] = 20011
+    indptr = np.concatenate([[0], np.cumsum(lens)])
+    x = g.integers(0, 3, int(indptr[-1]), dtype=np.uint8)
+    want, want_ip = M.segment_packbits(x != 0, indptr, bitorder)
+    buf = torch.full((len(want) + 32,), 0xA5, dtype=torch.uint8, device=cuda)
+    packed, new = ops.segment_packbits(torch.from_numpy(x).to(cuda), torch.from_numpy(indptr).to(cuda), bitorder,
+                                       out=buf[5:5 + len(want)])
+    got = buf.cpu().numpy()
+    assert np.array_equal(got[5:5 + len(want)], want)
+    assert (got[:5] == 0xA5).all() and (got[5 + len(want):] == 0xA5).all()
+    assert new.cpu().numpy().tolist() == want_ip.tolist()
+
+
 def _batch(seed, sizes, kinds):
     g = np.random.default_rng(seed)
     parents, ancs = [], []
