@@ -72,6 +72,11 @@ __device__ __forceinline__ void commit_status(const dft_commit_args& p, int b, i
 //   4 layers x 128 requests x 32 heads (2.1 GB)  368 / 380 / 584   367 / 366 / 374
 //   12 x 12 x 16 (302 MB)                         52 /  59 /  98    51 /  52 /  58
 //   batch 1, 24 x 32, into 2 snapshots, 16 nodes  65                34
+// Two corners are slower: one path node on a state that is in cache (24 layers
+// of batch 1 in place: 14.7 -> 15.8, where 4 nodes take 17.9 -> 16.6 and 16 38.8
+// -> 17.8), and tiles read element by element, whose kernel holds three
+// registers too many (the same with strided columns: 156 / 153 / 160 -> 162 /
+// 157 / 158; four waves per SIMD spill nothing and take 24% more at batch 32).
 // Five waves per SIMD (64 KiB of state in flight for each of five workgroups
 // per CU; four measured 4% slower); six leave 80 registers, spilled 2 and
 // took 381 us for the first row.
@@ -142,8 +147,8 @@ tree_commit_kernel(const CommitParams P) {
 
   // this lane's path entry, ahead of the tile (vector memory returns in order)
   // (the low word of an int64 entry: nodes are small, and a negative one's is negative)
-  const int node = static_cast<const int32_t*>(p.path)[((int64_t)b * p.path_req_stride + (lane < p.path_cols ? lane : 0)) *
-                                                      (p.path_dtype == DFT_I64 ? 2 : 1)];
+  const int64_t entry = (int64_t)b * p.path_req_stride + (lane < p.path_cols ? lane : 0);
+  const int node = static_cast<const int32_t*>(p.path)[entry * (p.path_dtype == DFT_I64 ? 2 : 1)];
   asm volatile("" ::: "memory");
 
   // ---- state tile: thread owns rows 16*rg .. 16*rg+15, cols 4*c4 .. 4*c4+3
@@ -185,7 +190,8 @@ tree_commit_kernel(const CommitParams P) {
   // of the copies, as every LDS read behind one is made to wait for it
   const int half = lane >> 5;
   const int mine = nodes[lane < T ? lane : 0];
-  const int copy0 = nodes[T > 0 ? min(2 * wave + half, T - 1) : 0], copy1 = nodes[T > 0 ? min(2 * wave + 8 + half, T - 1) : 0];
+  const int copy0 = nodes[T > 0 ? min(2 * wave + half, T - 1) : 0];
+  const int copy1 = nodes[T > 0 ? min(2 * wave + 8 + half, T - 1) : 0];
 
   // lane t: the weight of entry t, and whether it counts (an ancestor of u)
   const float* gl = p.gains + (int64_t)l * p.g_layer_stride + (int64_t)h * p.g_h_stride;

@@ -56,32 +56,24 @@ __global__ void __launch_bounds__(256) tree_conv_kernel(const dft_conv_args p) {
 
 // The plugin's layout (width 4, bf16 tokens / weights / output / window,
 // channel-contiguous rows) where the conv state is of another type or a tree
-// has more than 64 nodes; tree_conv4_rows_kernel below takes the rest, and
-// the figures here are of the time when this kernel took it all.  A block of one wave (64 threads)
-// covers 512 channels of one node; a thread owns 8 consecutive channels, so every
-// gathered token row, the weights (8 channels x 4 taps) and the output are
-// 16-byte accesses.  The gather columns are uniform over the block: the four
-// come in one batch of scalar loads (the index width is a template
-// parameter, so no load waits behind a dtype branch), the weights go out
-// meanwhile, and the four token loads are issued unconditionally (a tap
-// outside the tokens reads row 0 and is discarded).  Against a preamble of
-// dependent dtype-switched index loads this measured 41.0 -> 40.5 us.
-// The node's window over the block's channels is one contiguous run
-// (iw[n][c][0..2]): the threads' 48-byte pieces go through LDS so that each
-// store instruction writes 1 KiB of consecutive bytes (whole lines) instead
-// of 16 bytes every 48.
+// has more than 64 nodes (tree_conv4_rows_kernel below takes the rest).  A
+// workgroup of one wave covers 512 channels of one node; a thread owns 8
+// consecutive channels, so every gathered token row, the weights (8 channels x
+// 4 taps) and the output are 16-byte accesses.  The gather columns are uniform
+// over the workgroup: the four come in one batch of scalar loads (the index
+// width is a template parameter, so no load waits behind a dtype branch), the
+// weights go out meanwhile, and the four token loads are issued
+// unconditionally (a tap outside the tokens reads row 0 and is discarded).
+// The node's window over the channels is one contiguous run (iw[n][c][0..2]):
+// the threads' 48-byte pieces go through LDS so that each store instruction
+// writes 1 KiB of consecutive bytes (whole lines) instead of 16 bytes every 48.
 // The grid is 1-D and XCD-aware: workgroups are dealt to the 8 XCDs round
 // robin, so ids that agree mod 8 (one XCD, one L2) cover every node of one
 // (request, channel block) and the parents' rows re-read by the children
 // stay in that L2.
-// Measured at 64 requests x 32 nodes x 8192 channels: one node per block
-// beats blocks that walk 2-8 nodes (fewer, longer-lived waves) and beats
-// unstaged 48-byte window stores (non-temporal unstaged stores were slower
-// still: partial lines reach memory unmerged).  With the staged stores,
-// non-temporal y / window stores time the same as ordinary ones (within 1%).
-// Block size, in interleaved runs: one wave over 512 channels 40.0 us,
-// 128 threads over 1024 channels 40.8 us, 256 threads over 2048 channels
-// 41.3 us; 16 channels per thread (256 threads over 4096) 44.2 us.
+// us at 8192 channels with the window, here and on the per-channel kernel
+// above: 64 requests x 32 nodes with an fp32 conv state 44.0 / 160.2, 32 x 65
+// with a bf16 one 32.4 / 163.2, 1 x 96 5.8 / 10.6.
 // Request b's index (a slot) from an int32 or int64 array as two 32-bit
 // loads with no branch between them; idx NULL reads nothing (returns 0).
 __device__ __forceinline__ int64_t req_index(const void* idx, int dt, int b) {
@@ -141,11 +133,8 @@ __global__ void __launch_bounds__(64) tree_conv4_bf16_kernel(const dft_conv_args
     // Token rows: every load is issued (a tap outside the tokens reads row 0
     // and is discarded), so none waits on a branch.  A tap on a bf16 conv-state
     // column (a node within two edges of the root) gathers the column's 8
-    // values into the same registers instead, issued with the token loads:
-    // read through the per-element path below (8 two-byte loads per tap, each
-    // waited for in turn), these taps cost random 32-node trees about 5 us per
-    // launch at batch 64 (computing a chain's columns, which reach the state
-    // at 3 nodes only, ran 39.7 -> 34.7 us).
+    // values into the same registers instead, issued with the token loads
+    // (the per-element path below waits for 8 two-byte loads per tap in turn).
     const bool cs_bf16 = p.cs_dtype == DFT_BF16;
     u32x4 raw[4];
     bool tok[4], csg[4];
@@ -274,8 +263,8 @@ __global__ void __launch_bounds__(64 * W) tree_conv4_rows_kernel(const dft_conv_
   // them the row copies ahead of them) before the weights and the state were
   // asked for.  The arguments are forced into scalar registers first, for the
   // same reason.
-  asm volatile("" ::"s"(p.batch), "s"(p.n_nodes), "s"(p.channels), "s"(p.x), "s"(p.x_req_stride), "s"(p.x_node_stride), "s"(p.conv_state), "s"(p.cs_slot_stride),
-               "s"(p.cs_chan_stride), "s"(p.cs_col_stride), "s"(p.cs_indices), "s"(p.cs_indices_dtype), "s"(p.weight),
+  asm volatile("" ::"s"(p.batch), "s"(p.n_nodes), "s"(p.channels), "s"(p.x), "s"(p.x_req_stride),
+               "s"(p.x_node_stride), "s"(p.conv_state), "s"(p.cs_slot_stride), "s"(p.cs_chan_stride), "s"(p.cs_col_stride), "s"(p.cs_indices), "s"(p.cs_indices_dtype), "s"(p.weight),
                "s"(p.cidx), "s"(p.cidx_req_stride), "s"(p.cidx_node_stride), "s"(p.iw_indices), "s"(p.iw_indices_dtype),
                "s"(cblocks), "s"(splits));
   extern __shared__ u32x4 conv_lds[];
@@ -456,7 +445,7 @@ static bool launch_conv4_rows(const dft_conv_args* a, hipStream_t stream) {
   if (a->cs_dtype != DFT_BF16 || a->n_nodes > kConvNodes) return false;
   const int cblocks = (a->channels + kConvSlice - 1) / kConvSlice;
   const int64_t pairs8 = ((int64_t)a->batch * cblocks + 7) / 8;
-  if (pairs8 * 8 > (int64_t)0xffffffffll / (64 * 8)) return false;  // work-items in 32 bits (undivided: 256 pairs or more)
+  if (pairs8 * 8 > (int64_t)0xffffffffll / (64 * 8)) return false;  // work-items in 32 bits
   if (a->n_nodes <= 2)
     launch_rows_kernel<2>(a, cblocks, pairs8, stream);
   else if (a->n_nodes <= 4 || (a->n_nodes <= 12 && pairs8 * 8 >= kConvPairs))

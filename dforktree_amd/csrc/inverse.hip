@@ -103,7 +103,8 @@ __device__ __forceinline__ void block_rows(float* a, int n16, int g4, f32x4 (&xr
     if constexpr (I > 0) {
       f32x4 am[I];  // A[16I + n][16m + 4g ..]
 #pragma unroll
-      for (int m = 0; m < I; ++m) am[m] = *reinterpret_cast<const f32x4*>(&a[mat_at<NP>(16 * I + n16, 16 * m + 4 * g4)]);
+      for (int m = 0; m < I; ++m)
+        am[m] = *reinterpret_cast<const f32x4*>(&a[mat_at<NP>(16 * I + n16, 16 * m + 4 * g4)]);
 #pragma unroll
       for (int j = 0; j < I; ++j) {
         x[j] = f32x4{};

@@ -1,5 +1,5 @@
 // Tree structure from parent indices (tree_ops.py:68-89, fc1_builder.py:38-47).
-// One workgroup of four waves per request (n <= 64 nodes, lane i = node i):
+// Four waves per request, or one (n <= 64 nodes, lane i = node i):
 //   - ancestor-or-self set of i as a uint64 (exact closure by pointer
 //     doubling: after k rounds the set holds the ancestors at distances below
 //     2^k and p the 2^k-th one, so six rounds cover any tree; the reference's
@@ -13,11 +13,12 @@
 //
 // Bound by the chain of one request: every wave forms the sets (registers
 // and lane shuffles), then wave 0 writes the sets, depths and status, wave 1
-// cidx, wave 2 the links, and all four the dense rows.  128 requests of 8-64
-// nodes with every output: 20.4 us with one wave per request that walked the
-// parents one LDS read at a time (63 for a chain) and searched the links by
-// a loop over the nodes, now 4.7 us, 6.4 with what no tree covers zeroed too
-// (two fill launches fewer).
+// cidx, wave 2 the links, and all four the dense rows (one wave does it all
+// where there is little to share out: launch_tree_struct).  128 requests of
+// 8-64 nodes with every output: 19.9 us with one wave per request that walked
+// the parents one LDS read at a time (63 for a chain) and searched the links
+// by a loop over the nodes, now 4.2 us, 4.6 with what no tree covers zeroed
+// too (23.6 with two fill launches ahead).
 #include "dft_device.h"
 
 namespace dft {
@@ -109,7 +110,8 @@ __device__ __forceinline__ void tree_of_request(const dft_tree_args& p, int b, i
     const uint32_t lo = (uint32_t)bits, hi = (uint32_t)(bits >> 32);
     const int rows = FILL ? p.n_nodes : n, cols = rows;
     for (int r = w; r < rows; r += W) {  // (uniform)
-      uint64_t rb = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, r) << 32) | (uint32_t)__builtin_amdgcn_readlane(lo, r);
+      uint64_t rb = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, r) << 32) |
+                    (uint32_t)__builtin_amdgcn_readlane(lo, r);
       if (FILL && r >= n) rb = 0;
       if (lane < cols) base[(int64_t)r * p.anc_row_stride + lane] = (float)((rb >> lane) & 1ull);
     }
@@ -119,7 +121,8 @@ __device__ __forceinline__ void tree_of_request(const dft_tree_args& p, int b, i
 }
 
 // The smallest and the largest of the batch's cu_seqlens (every request's
-// rows lie between them).
+// rows lie between them), reduced in registers (one LDS atomic per request
+// was 15 us at 1024 requests, 129 at 8192, ahead of what it is for).
 __device__ __forceinline__ void packed_ends(const dft_tree_args& p, int& lo, int& hi) {
   __shared__ int ends[2][4];
   const int wave = threadIdx.x >> 6;
