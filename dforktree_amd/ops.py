@@ -106,7 +106,8 @@ def tree_verify(y: torch.Tensor, a: torch.Tensor, b: torch.Tensor, A_log: Option
     request longer than n_nodes is cut to n_nodes rows (DFT_STATUS_SPAN).
     ``size_order``: the records ``size_order(cu_seqlens, n_nodes)`` wrote for
     this packed batch (once per step, shared by every layer); a launch split
-    by tree size then runs each class's requests first in its kernel.
+    by tree size then takes the large trees first, as one kernel with an even
+    hv, else as two that each take their own class's requests first.
     """
     args, o, dev, _keep = _verify_args(
         y, a, b, A_log, dt_bias, state, hk=hk, hv=hv, anc=anc, anc_bits=anc_bits, batch=batch, n_nodes=n_nodes,
